@@ -27,6 +27,7 @@
 
 #include "z4c_adjoint.hpp"
 #include "z4c_device.hpp"
+#include "z4c_fused.hpp"
 #include "z4c_mesh.hpp"
 #include "z4c_mi355x.h"
 #include "z4c_refine.hpp"
@@ -387,102 +388,189 @@ __global__ void __launch_bounds__(TILE) k_algconstr(AlgArgs a) {
                   a.tf_force, a.force_reg);
 }
 
-// ---------------------------------------------------------------------------
-// Fused bt_rk4 stage: RHS assembly + stage update + AlgConstr at interior
-// vertices.  The reference runs CalculateZ4cRHS, IntegrateZ4c (SumBT over the
-// registers) and EnforceAlgConstr as separate tasks
-// (src/task_list/gr/task_list_gr_z4c.cpp:46-64); the update of each variable
-// is pointwise, so it is formed as soon as the variable's right-hand side is,
-// with the same sums in the same order:
-//   u_{s+1} = u_n + (A[s+1][s] dt) k_s          (the one nonzero of bt_rk4's row)
-//   acc_1 = u_n + (b_1 dt) k_1,  acc_s = acc_{s-1} + (b_s dt) k_s
-//   u_{n+1} = acc_3 + (b_4 dt) k_4 = ((u_n + b_1 dt k_1) + b_2 dt k_2) + ...
-// followed by AlgConstr of the point (src/z4c/z4c.cpp:677-991).
-// ---------------------------------------------------------------------------
-struct StageArgs {
-  RhsArgs r;         // r.u: stage input state (read only); r.rhs unused
-  const double* un;  // state at the start of the step (unused at the last stage)
-  int un_int;        // un is interior-indexed (the kept copy) instead of a state
-  double* acc;       // running sum of the final combination (interior-indexed)
-  double* out;       // stage output state (the caller's state at the last stage)
-  double* keep;      // stage 1 of the in-place step: receives u_n, interior-
-                     // indexed (else null)
-  double wa, wb;     // A[s+1][s] * dt and b_s * dt
-  int stage;         // 1..4
-  int cowling;
-  double eps_floor;
-  int tf_force, force_reg;
-  // low-storage stage (k_rk4_stage<..., true>): u1 register (interior-
-  // indexed) and the stage's delta, gamma_1, gamma_2 and beta * dt
-  double* u1;
-  double ls_w[4];
-  int ls_last;       // the last stage: u1 is not stored
-};
-
-// The curvature part (Ricci, D_aD_b alpha) is formed in the same kernel and
-// staged in LDS (a per-thread column) instead of a separate pass through HBM.
 // The stage kernel's state stores are streaming (non-temporal): the next
 // pass reads them back from HBM in any case.
 __device__ __forceinline__ void st_state(double* p, double v) { __builtin_nontemporal_store(v, p); }
 
-// ALG: AlgConstr at the end (the step with ghosts held at u_n); without it
-// the stage leaves the sums for the ghost update and the whole-block
-// AlgConstr that follow it, in the task list's order.  LS: the update is a
-// low-storage 2S stage instead of bt_rk4's (see below).
-template <bool WITH_SOMMERFELD, bool ALG, bool LS = false>
-__global__ void __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(2)))
-k_rk4_stage(StageArgs a) {
-  __shared__ double ko[NVAR * TILE];  // this point's k_s, staged (see k_rhs_alg)
-  __shared__ double cvs[12 * TILE];   // this point's curvature part
-  int b, i, j, k;
-  if (!tile_point(a.r.L, b, i, j, k)) return;
-  const int t = threadIdx.x;
-  const DevBlock B = a.r.blocks[b];
-  const int N = B.npts;
-  const int p = flat(B, i, j, k);
-  const long long base = B.off * NVAR;
-  const int qi = (i - B.il) + B.ni * ((j - B.jl) + B.nj * (k - B.kl));
-  if (a.cowling) {
-    for (int n = 0; n < NVAR; ++n) ko[n * TILE + t] = 0.0;
-  } else {
-    const PointIO X = point_io(a.r, B, p, qi);
-    rhs_curvature_point(a.r.o, X, [&](int n, double v) { cvs[n * TILE + t] = v; });
-    rhs_assembly_point(a.r.o, X, [&](int n) { return cvs[n * TILE + t]; },
-                       [&](int n, double v) { ko[n * TILE + t] = v; });
-    if (WITH_SOMMERFELD && B.faces && on_sommerfeld_face(B, i, j, k)) {
-      const Pt P = make_pt(p, B.nn1, B.nn2, N);
-      sommerfeld_point(B, X.U, P, a.r.u + base, i, j, k, N,
-                       [&](int n, double v) { ko[n * TILE + t] = v; });
+// Right-hand side of a brick (z4c_fused.hpp), stored as such or taken into the
+// stage update.  The reference runs CalculateZ4cRHS, IntegrateZ4c (SumBT over
+// the registers) and EnforceAlgConstr as separate tasks
+// (src/task_list/gr/task_list_gr_z4c.cpp:46-64); the update is pointwise, so
+// every variable's follows its right-hand side, with the same sums in the same
+// order:
+//   u_{s+1} = u_n + (A[s+1][s] dt) k_s          (the one nonzero of bt_rk4's row)
+//   acc_1 = u_n + (b_1 dt) k_1,  acc_s = acc_{s-1} + (b_s dt) k_s
+//   u_{n+1} = acc_3 + (b_4 dt) k_4 = ((u_n + b_1 dt k_1) + b_2 dt k_2) + ...
+// followed by AlgConstr of the point (src/z4c/z4c.cpp:677-991).  LS: the
+// low-storage 2S stage (task_list_gr_z4c.cpp:176-193) with WeightedAve_'s case
+// split (weighted_ave.cpp:21-132):
+//   u1 = WeightedAve(u1, u, -, {1, delta, 0})   (u1 = 0 before stage 1)
+//   u  = WeightedAve(u, u1, -, {gamma_1, gamma_2, 0}) + (beta dt) rhs
+// The running sum, the kept u_n and u1 are interior-indexed (whole 128-byte
+// lines of interior points).
+template <class C>
+__global__ void __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(2)))
+k_fused(FusedArgs args) {
+  __shared__ __align__(16) double winA[C::WIN];
+  __shared__ __align__(16) double winB[C::WIN];
+  __shared__ double der[C::NDY + C::NDZ];
+  __shared__ double cols[C::NCOL * C::THREADS];
+  __shared__ int halo[(C::HROUNDS + 1) * C::THREADS];
+  const KernArgs<FusedArgs> ka;
+  const int G = gridDim.x;  // multiple of 8: XCD-contiguous ranges
+  const int t = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
+  if (t >= args.ntiles) return;
+  const int tid = threadIdx.x;
+  auto col = [&](int c) -> double& { return cols[c * C::THREADS + tid]; };
+  double kK = 0.0, kT = 0.0, kal = 0.0, kb[3] = {}, kg[6] = {}, kA[6] = {};
+  {
+    const auto& a = args;
+    const FusedTile T = a.tiles[t];
+    const DevBlock& B = a.blocks[T.block];
+    const int N = B.npts;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int tx, ty, tz;
+    const bool in = fused_vertex<C>(T, tid, tx, ty, tz);
+    const double* u = a.u + B.off * NVAR;
+    FusedPoint<C> P;
+    P.ub = u;
+    P.N = __builtin_amdgcn_readfirstlane(N);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      // lidx equals cidx1
+      P.c1[d] = uniform(B.cidx1[d]);
+      P.c2[d] = uniform(B.cidx2[d]);
+      P.cd[d] = uniform(B.cidxd[d]);
+    }
+    P.win[0] = winA;
+    P.win[1] = winB;
+    P.der = der;
+    P.halo = halo + tid;
+    P.wave = wave;
+    {
+      const int row0 = wave * C::RPI + lane / C::LPR, c0 = 2 * (lane % C::LPR);
+      int kk = row0 / C::PY, jj = row0 - kk * C::PY;
+      P.step0 = 8 * B.nn1 * (C::STEP / C::PY * B.nn2 + C::STEP % C::PY);
+      P.step1 = 8 * B.nn1 * (B.nn2 - C::PY);
+      P.voff0 = 8u * (unsigned)((B.il + T.i0 - 4 + c0) +
+                                B.nn1 * ((B.jl + T.j0 - 4 + jj) + B.nn2 * (B.kl + T.k0 - 4 + kk)));
+      P.bits = lane >= C::LPR * C::RPI ? 1u << 31 : 0u;
+      // the pair's nearest distance from the brick along x
+      const int dx = c0 + 1 < 4 ? 3 - c0 : max(0, c0 - T.ni - 3);
+#pragma unroll
+      for (int r = 0; r < C::ROUNDS; ++r) {
+        // the row's distances in y and z; a field needs the vertices that lie
+        // off the brick along one axis (by up to 4) and, with mixed
+        // derivatives, along two (by up to 3)
+        const int dy = jj < 4 ? 4 - jj : max(0, jj - T.nj - 3);
+        const int dz = kk < 4 ? 4 - kk : max(0, kk - T.nk - 3);
+        const int off = (dx > 0) + (dy > 0) + (dz > 0);
+        const int far = max(dx, max(dy, dz));
+        const bool star = off <= 1 && far <= 4;
+        const bool need = star || (off == 2 && far <= 3);
+        const bool wrap = jj + C::STEP % C::PY >= C::PY;
+        P.bits |= (need ? 0u : 1u << r) | (star ? 0u : 1u << (10 + r)) | (wrap ? 1u << (20 + r) : 0u);
+        jj += C::STEP % C::PY - (wrap ? C::PY : 0);
+        kk += C::STEP / C::PY + (wrap ? 1 : 0);
+      }
+    }
+    P.o = (tx + 4) + C::PX * (ty + 4) + C::PLANE * (tz + 4);
+    halo[C::HROUNDS * C::THREADS + tid] =
+        ((tx + 3) + C::DX * (ty + C::BY * tz)) |
+        ((C::NDY + (tx + 3) + C::DX * (ty + 3) + C::DZP * tz) << 16);
+#pragma unroll
+    for (int r = 0; r < C::HROUNDS; ++r) {
+      const int s = r * C::WAVES + wave;
+      int x, y, z;
+      bool ok;
+      if (s < 2 * C::SX) {
+        const int e = (s < C::SX ? s : s - C::SX) * 64 + lane;
+        const int hx = e % 6;
+        x = hx < 3 ? hx - 3 : T.ni + hx - 3;
+        y = e / 6 % C::BY;
+        z = e / (6 * C::BY);
+        ok = e < C::HX;
+      } else {
+        const int e = (s - 2 * C::SX) * 64 + lane;
+        const int hy = e / C::BX % 6;
+        x = e % C::BX;
+        y = hy < 3 ? hy - 3 : T.nj + hy - 3;
+        z = e / (6 * C::BX);
+        ok = e < C::HY;
+      }
+      const int src = ok ? (x + 4) + C::PX * (y + 4) + C::PLANE * (z + 4) : P.o;
+      const int dst = !ok ? -1
+                          : (s < C::SX ? (x + 3) + C::DX * (y + C::BY * z)
+                                       : C::NDY + (x + 3) + C::DX * (y + 3) + C::DZP * z);
+      halo[r * C::THREADS + tid] = src | (dst * 65536);
+    }
+    P.p8 = in ? 8u * (unsigned)flat(B, B.il + T.i0 + tx, B.jl + T.j0 + ty, B.kl + T.k0 + tz)
+              : DV_DROP;
+    P.dst = (a.rhs ? a.rhs : a.out) + B.off * NVAR;
+    P.diss = a.o.diss;
+    P.bx = P.at(V_BETAX);
+    P.by = P.at(V_BETAX + 1);
+    P.bz = P.at(V_BETAX + 2);
+    if (!a.cowling) P.template fetch<fu_field(0), 0>();
+    if (!a.cowling) {
+      fused_rhs<C>(P, ka, a.mat ? a.mat + B.off * NMAT : nullptr, col, kK, kT, kal, kb,
+                   kg, kA);
+    } else {
+#pragma unroll
+      for (int c = 0; c < C::NCOL; ++c) col(c) = 0.0;
     }
   }
-  // stage update of every variable, then AlgConstr of the point.  The
-  // running sum and the kept u_n are interior-indexed (whole 128-byte lines
-  // of interior points, no ghost columns in the lines read).
-  const long long ibase = B.ioff * NVAR;
-  const double* un = a.un_int ? a.un + ibase : a.un + base;
-  double* acc = a.acc + ibase;
-  double* out = a.out + base;
-  double* keep = a.keep ? a.keep + ibase : nullptr;
-  const int stage = a.stage;
-  const double wa = a.wa, wb = a.wb;
+  // the tile again (nothing of it is held through the fields)
+  const auto& a = ka.get();
+  int t2 = t;
+  asm volatile("" : "+v"(t2));
+  const FusedTile T = a.tiles[__builtin_amdgcn_readfirstlane(t2)];
+  const DevBlock& B = a.blocks[T.block];
+  int tx, ty, tz;
+  if (!fused_vertex<C>(T, tid, tx, ty, tz)) return;
+  const int N = B.npts;
+  const int i = B.il + T.i0 + tx, j = B.jl + T.j0 + ty, k = B.kl + T.k0 + tz;
+  const int p = flat(B, i, j, k);
+  const long long base = B.off * NVAR;
+  const double* u = a.u + base + p;
+  auto kv = [&](int n) -> double& {
+    if (n == V_CHI) return col(3);
+    if (n >= V_GXX && n < V_GXX + 6) return kg[n - V_GXX];
+    if (n == V_KHAT) return kK;
+    if (n >= V_AXX && n < V_AXX + 6) return kA[n - V_AXX];
+    if (n >= V_GAMX && n < V_GAMX + 3) return col(n - V_GAMX);
+    if (n == V_THETA) return kT;
+    if (n == V_ALPHA) return kal;
+    return kb[n - V_BETAX];
+  };
+  if (a.sommerfeld && !a.cowling && B.faces && on_sommerfeld_face(B, i, j, k)) {
+    const Pt P = make_pt(p, B.nn1, B.nn2, N);
+    sommerfeld_point(B, make_buf(a.u + base, (long long)NVAR * N * 8), P, a.u + base, i, j, k, N,
+                     [&](int n, double v) { kv(n) = v; });
+  }
+  if (a.rhs) {
+    double* rhs = a.rhs + base + p;
+#pragma unroll
+    for (int n = 0; n < NVAR; ++n) rhs[(long long)n * N] = kv(n);
+    return;
+  }
+  const int qi = (i - B.il) + B.ni * ((j - B.jl) + B.nj * (k - B.kl));
+  const long long ibase = B.ioff * NVAR + qi;
   const int NI = B.nint;
+  double* out = a.out + base + p;
+  double* acc = a.acc + ibase;
+  const int stage = a.stage;
   double s[NVAR];
-  if (LS) {
-    // IntegrateZ4c's low-storage branch (task_list_gr_z4c.cpp:176-193) at
-    // this vertex, with WeightedAve_'s case split (weighted_ave.cpp:21-132):
-    //   u1 = WeightedAve(u1, u, -, {1, delta, 0})   (u1 = 0 before stage 1)
-    //   u  = WeightedAve(u, u1, -, {gamma_1, gamma_2, 0})
-    //   u += (beta dt) rhs                          (AddZ4cRHS)
-    const double* uin = a.r.u + base;
-    double* u1 = a.u1 + ibase;
+  if (a.ls) {
+    double* u1 = acc;
     const double dl = a.ls_w[0], g1 = a.ls_w[1], g2 = a.ls_w[2], bdt = a.ls_w[3];
 #pragma unroll
     for (int n = 0; n < NVAR; ++n) {
-      const int ei = n * NI + qi;
-      const double u0 = uin[n * N + p];
-      double v1 = (stage == 1) ? 0.0 : u1[ei];
+      const double u0 = u[(long long)n * N];
+      double v1 = (stage == 1) ? 0.0 : u1[(long long)n * NI];
       if (dl != 0.0) v1 += dl * u0;
-      if (!a.ls_last) st_state(u1 + ei, v1);
+      if (!a.ls_last) st_state(u1 + (long long)n * NI, v1);
       double v;
       if (g1 == 1.0)
         v = (g2 != 0.0) ? u0 + g2 * v1 : u0;
@@ -490,34 +578,44 @@ k_rk4_stage(StageArgs a) {
         v = (g2 == 1.0) ? v1 : g2 * v1;
       else
         v = (g2 != 0.0) ? g1 * u0 + g2 * v1 : u0 * g1;
-      s[n] = v + bdt * ko[n * TILE + t];
+      s[n] = v + bdt * kv(n);
     }
-  } else
+  } else {
+    const double wa = a.wa, wb = a.wb;
+    const double* un = a.un_int ? a.un + ibase : a.un + base + p;
+    const long long un_st = a.un_int ? NI : N;
+    double* keep = a.keep ? a.keep + ibase : nullptr;
+    // every load before the first store: one wait instead of one per field
+    double x[NVAR];
+    if (stage < 4) {
 #pragma unroll
-  for (int n = 0; n < NVAR; ++n) {
-    const int e = n * N + p;
-    const int ei = n * NI + qi;
-    const int eu = a.un_int ? ei : e;
-    const double kv = ko[n * TILE + t];
-    if (stage == 1) {
-      const double u0 = un[eu];
-      if (keep) st_state(keep + ei, u0);
-      st_state(acc + ei, u0 + wb * kv);
-      s[n] = u0 + wa * kv;
-    } else if (stage < 4) {
-      st_state(acc + ei, acc[ei] + wb * kv);
-      s[n] = un[eu] + wa * kv;
-    } else {
-      s[n] = acc[ei] + wb * kv;
+      for (int n = 0; n < NVAR; ++n) s[n] = un[n * un_st];
+    }
+    if (stage > 1) {
+#pragma unroll
+      for (int n = 0; n < NVAR; ++n) x[n] = acc[(long long)n * NI];
+    }
+#pragma unroll
+    for (int n = 0; n < NVAR; ++n) {
+      const double v = kv(n);
+      if (stage == 1) {
+        if (keep) st_state(keep + (long long)n * NI, s[n]);
+        st_state(acc + (long long)n * NI, s[n] + wb * v);
+        s[n] = s[n] + wa * v;
+      } else if (stage < 4) {
+        st_state(acc + (long long)n * NI, x[n] + wb * v);
+        s[n] = s[n] + wa * v;
+      } else {
+        s[n] = x[n] + wb * v;
+      }
     }
   }
-  if (ALG)
+  if (a.alg)
     algconstr_vals(s + V_GXX, s + V_AXX, s[V_CHI], s[V_ALPHA], a.eps_floor, a.tf_force,
                    a.force_reg);
 #pragma unroll
-  for (int n = 0; n < NVAR; ++n) st_state(out + n * N + p, s[n]);
+  for (int n = 0; n < NVAR; ++n) st_state(out + (long long)n * N, s[n]);
 }
-
 // Ghost vertices of a fused step with ghosts held at u_n: what the unfused
 // sequence leaves there after every stage is AlgConstr(u_n + 0), so the step
 // applies AlgConstr to the state's ghosts once (after the first stage has
@@ -578,12 +676,8 @@ __global__ void __launch_bounds__(TILE) k_rk4_ghosts(GhostArgs a) {
     u[V_ALPHA * N + p] = s[V_ALPHA];
   }
   double* w0 = a.w0 + base;
-  double* w1 = a.w1 + base;
 #pragma unroll
-  for (int n = 0; n < NVAR; ++n) {
-    w0[n * N + p] = s[n];
-    w1[n * N + p] = s[n];
-  }
+  for (int n = 0; n < NVAR; ++n) w0[n * N + p] = s[n];
 }
 
 // ---------------------------------------------------------------------------
@@ -2658,6 +2752,11 @@ struct z4c_ctx {
   int lin_ntiles = 0;
   int st_ntiles[NSTCFG] = {};
   long long total_int = 0;  // interior points
+  long long total_dv = 0;   // doubles of the derivative slots (dv, allocated on first use)
+  FusedTile* fu_tiles = nullptr;  // bricks of the one-kernel right-hand side
+  int fu_ntiles = 0;
+  bool small = false;       // too little work to fill the chip with bricks (launch_rhs)
+  bool two_pass = false;    // z4c_rhs in two passes (a stencil workgroup size was fixed)
   double* snap = nullptr;  // periodic-fill snapshot / exchange scratch (lazy)
   long long snap_elems = 0;
   double* hst = nullptr;   // history partial sums (lazy)
@@ -2798,6 +2897,7 @@ struct z4c_ctx {
   struct TimedLaunch {
     int pass;
     hipEvent_t a, b;
+    double part;  // share of the launch's time that counts for the pass
   };
   bool timing = false;
   std::vector<TimedLaunch> tev;
@@ -2871,6 +2971,10 @@ struct z4c_ctx {
     hipFree(lin_tiles);
     lin_tiles = nullptr;
     lin_ntiles = 0;
+    hipFree(fu_tiles);
+    fu_tiles = nullptr;
+    fu_ntiles = 0;
+    two_pass = false;
     hipFree(snap);
     hipFree(hst);
     hst = nullptr;
@@ -2919,7 +3023,9 @@ struct PassTimer {
   int pass;
   hipStream_t s;
   hipEvent_t a = nullptr;
-  PassTimer(z4c_ctx* c_, int pass_, hipStream_t s_) : c(c_), pass(pass_), s(s_) {
+  double part;
+  PassTimer(z4c_ctx* c_, int pass_, hipStream_t s_, double part_ = 1.0)
+      : c(c_), pass(pass_), s(s_), part(part_) {
     if (c->timing && hipEventCreate(&a) == hipSuccess) hipEventRecord(a, s);
   }
   ~PassTimer() {
@@ -2930,7 +3036,7 @@ struct PassTimer {
       return;
     }
     hipEventRecord(b, s);
-    c->tev.push_back({pass, a, b});
+    c->tev.push_back({pass, a, b, part});
   }
 };
 
@@ -3082,8 +3188,66 @@ void launch_stencil_cfg(int cfg, const StencilArgs& sa, hipStream_t s) {
   }
 }
 
+// The derivative slots, allocated by the first two-pass right-hand side.
+int ensure_slots(z4c_ctx* c) {
+  if (c->dv) return Z4C_OK;
+  if (hipMalloc(&c->dv, sizeof(double) * c->total_dv) != hipSuccess) {
+    c->dv = nullptr;
+    return fail(Z4C_ENOMEM, "derivative-slot allocation failed");
+  }
+  return Z4C_OK;
+}
+
+// Bricks of the one-kernel right-hand side, cut as equal as they divide.
+int build_fused_tiles(z4c_ctx* c, const std::vector<DevBlock>& hb) {
+  constexpr int M[3] = {FuCfg::BX, FuCfg::BY, FuCfg::BZ};
+  std::vector<FusedTile> t;
+  int planes = 0;
+  for (int b = 0; b < (int)hb.size(); ++b) {
+    const int n[3] = {hb[b].ni, hb[b].nj, hb[b].nk};
+    planes = std::max(planes, n[2]);
+    int s[3];
+    for (int d = 0; d < 3; ++d) {
+      const int q = (n[d] + M[d] - 1) / M[d];
+      s[d] = (n[d] + q - 1) / q;
+    }
+    for (int k0 = 0; k0 < n[2]; k0 += s[2])
+      for (int j0 = 0; j0 < n[1]; j0 += s[1])
+        for (int i0 = 0; i0 < n[0]; i0 += s[0])
+          t.push_back(FusedTile{b, i0, j0, k0, std::min(s[0], n[0] - i0), std::min(s[1], n[1] - j0),
+                                std::min(s[2], n[2] - k0)});
+  }
+  if (hipMalloc(&c->fu_tiles, sizeof(FusedTile) * t.size()) != hipSuccess)
+    return fail(Z4C_ENOMEM, "set_blocks: brick table allocation failed");
+  HIPCALL(hipMemcpy(c->fu_tiles, t.data(), sizeof(FusedTile) * t.size(), hipMemcpyHostToDevice));
+  c->fu_ntiles = (int)t.size();
+  // The one-kernel form runs a brick's 22 fields in turn (37 us however few
+  // the bricks); the two passes split a block by field as well and march its
+  // planes.  Measured on one block: 31.7 / 34.5 / 38.0 / 41.5 us in two passes
+  // for 7 / 9 / 11 / 13 vertices a side against 37-39 us, and 30.7 against 37.3
+  // us for 16 blocks of 9^3 (96 bricks), 71.7 against 53.7 us for 64 (384).
+  c->small = t.size() <= 128 && planes <= 10;
+  return c->small ? ensure_slots(c) : Z4C_OK;
+}
+
+// The launch does the work of the stencil and the assembly passes: the kernel
+// timer divides its time between them by their arithmetic (4435 and 3374
+// operations per vertex).
+int launch_fused(z4c_ctx* c, FusedArgs a, hipStream_t s) {
+  a.blocks = c->d_blocks;
+  a.tiles = c->fu_tiles;
+  a.ntiles = c->fu_ntiles;
+  PassTimer t1(c, Z4C_PASS_STENCIL, s, 0.57);
+  PassTimer t2(c, Z4C_PASS_ASSEMBLY, s, 0.43);
+  hipLaunchKernelGGL(k_fused<FuCfg>, dim3(grid_for(a.ntiles)), dim3(FuCfg::THREADS), 0, s, a);
+  HIPCALL(hipGetLastError());
+  return Z4C_OK;
+}
+
 // The stencil pass over all blocks: one launch per configuration in use.
 int launch_stencil(z4c_ctx* c, const double* u, const z4c_params* p, hipStream_t s) {
+  const int rc = ensure_slots(c);
+  if (rc) return rc;
   PassTimer t(c, Z4C_PASS_STENCIL, s);
   for (int q = 0; q < NSTCFG; ++q) {
     if (!c->st_ntiles[q]) continue;
@@ -3098,6 +3262,19 @@ int launch_stencil(z4c_ctx* c, const double* u, const z4c_params* p, hipStream_t
 int launch_rhs(z4c_ctx* c, const z4c_params* p, const double* u,
                const double* mat, double* rhs, bool sommerfeld, hipStream_t s) {
   if (p->cowling) return fill(c, rhs, 0.0, c->total_pts * NVAR, s);
+  // one kernel, unless the batch is small or the right-hand side is written
+  // over its own input (every brick reads its neighbours' vertices)
+  const long long nn = c->total_pts * NVAR;
+  const bool apart = (uintptr_t)rhs + 8 * nn <= (uintptr_t)u || (uintptr_t)u + 8 * nn <= (uintptr_t)rhs;
+  if (apart && !c->two_pass && !c->small) {
+    FusedArgs a{};
+    a.u = u;
+    a.mat = mat;
+    a.o = rhs_params(p);
+    a.sommerfeld = sommerfeld;
+    a.rhs = rhs;
+    return launch_fused(c, a, s);
+  }
   int rc = launch_stencil(c, u, p, s);
   if (rc) return rc;
   RhsArgs a{c->d_blocks, launch_of(c, BOX_INTERIOR), u, c->dv, mat, rhs, rhs_params(p)};
@@ -3985,12 +4162,13 @@ int z4c_set_blocks(z4c_ctx* c, const z4c_block* blocks, int nblocks,
     return fail(Z4C_ENOMEM, "set_blocks: derivative storage allocation failed");
   // prepared derivatives start at zero (the reference zero-initialises them)
   HIPCALL(hipMemset(c->d1, 0, sizeof(double) * off * ND1));
-  if (hipMalloc(&c->dv, sizeof(double) * doff) != hipSuccess)
-    return fail(Z4C_ENOMEM, "set_blocks: derivative-slot allocation failed");
+  c->total_dv = doff;
   c->blk_cfg = blk_cfg;
   c->hdev = hb;
   {
     int rc = build_stencil_plan(c, hb);
+    if (rc) return rc;
+    rc = build_fused_tiles(c, hb);
     if (rc) return rc;
     rc = build_physical_tables(c, hb);
     if (rc) return rc;
@@ -4808,6 +4986,9 @@ int z4c_autotune(z4c_ctx* c, const z4c_params* p, const double* u, int reps, voi
   int rc = check_ctx(c);
   if (rc) return rc;
   if (!p || !u || reps < 1) return fail(Z4C_EINVAL, "autotune: bad argument");
+  rc = ensure_slots(c);
+  if (rc) return rc;
+  c->two_pass = false;
   hipStream_t s = (hipStream_t)stream;
   std::map<std::array<int, 3>, std::vector<int>> classes;
   for (int b = 0; b < c->nblocks; ++b)
@@ -4878,6 +5059,7 @@ int z4c_set_stencil_threads(z4c_ctx* c, int block, int threads) {
       return fail(Z4C_EINVAL, "set_stencil_threads: no tile of that size fits block " +
                                   std::to_string(b));
   for (int b = b0; b < b1; ++b) c->blk_cfg[b] = q;
+  c->two_pass = true;
   return build_stencil_plan(c, c->hdev);
 }
 
@@ -4911,7 +5093,7 @@ int z4c_get_timing(z4c_ctx* c, double* ms_total, long long* launches, int npass)
       break;
     }
     if (t.pass >= 0 && t.pass < npass) {
-      ms_total[t.pass] += ms;
+      ms_total[t.pass] += t.part * ms;
       launches[t.pass] += 1;
     }
   }
@@ -4922,6 +5104,16 @@ int z4c_get_timing(z4c_ctx* c, double* ms_total, long long* launches, int npass)
 }  // extern "C"
 
 namespace {
+int ghost_update(z4c_ctx* c, double* u, int ghosts, hipStream_t s) {
+  int rc = Z4C_OK;
+  if (ghosts & 1)
+    rc = launch_periodic(c, NVAR, u, s);
+  else if (ghosts & 2)
+    rc = launch_exchange(c, NVAR, u, s);
+  if (!rc && (ghosts & 4)) rc = launch_physical(c, NVAR, u, s);
+  return rc;
+}
+
 // ghosts: 0 holds the ghosts at u_n (AlgConstr(u_n), formed once); else the
 // ghost update of z4c_rk4_stage after every stage (1 single-block periodic
 // fill or 2 the exchange, plus 4 the physical fill), on the stage state whose
@@ -4936,97 +5128,57 @@ int launch_rk4_step(z4c_ctx* c, const z4c_params* p, double dt, double* u, doubl
   // bt_rk4 (task_list_integrators_butcher.cpp:37-49): subdiagonal of A and b
   static const double Asub[4] = {0.5, 0.5, 1.0, 0.0};
   static const double Bw[4] = {1. / 6., 1. / 3., 1. / 3., 1. / 6.};
-  // In place (no Sommerfeld face): every stage state overwrites the
-  // interior of u (the stage kernel reads u only at its own point), u_n is
-  // kept in W0 by stage 1, and u's ghosts, AlgConstr(u_n) after stage 1, are
-  // the ghosts of every later stage.  With Sommerfeld faces the stage reads
-  // neighbouring values of its input, so the stage states alternate between
-  // W0 and W1 and the ghosts are copied into both.
-  bool faces = false;
-  for (const DevBlock& B : c->hdev) faces = faces || B.faces != 0;
-  const bool inplace = !faces;
-  double* const ins[4] = {u, W0, W1, W0};
-  double* const outs[4] = {W0, W1, W0, u};
-  // with a ghost update, u_n's ghosts (what SumBT leaves at the ghosts) are
-  // kept in W1 when the stages run in place; otherwise u keeps them
-  const GhostArgs keep_ghosts{c->d_blocks, launch_of(c, BOX_GHOST), u, W1, nullptr,
-                              p->eps_floor, p->tf_force_regularization,
-                              p->force_regularization};
+  // Every stage reads its neighbours' vertices, so no stage overwrites its
+  // input.  With ghosts held at u_n the states alternate between W0 and u
+  // (u_n is kept interior-indexed in W1), and both hold the ghosts
+  // AlgConstr(u_n) once stage 1 has read u_n's.  With a ghost update the
+  // first three states alternate between W0 and W1, and u keeps u_n and its
+  // ghosts until the last stage.
+  double* const ins[4] = {u, W0, ghosts ? W1 : u, W0};
+  double* const outs[4] = {W0, ghosts ? W1 : u, W0, u};
   // the ghost update across levels writes every ghost (zero, then the
   // contributions): u_n's ghosts need no keeping
   const bool all_ghosts = (ghosts & 2) && c->ml;
-  if (ghosts && inplace && !all_ghosts) {
-    PassTimer t(c, Z4C_PASS_GHOSTS, s);
-    hipLaunchKernelGGL(k_ghost_copy, dim3(grid_for(keep_ghosts.L.ntiles)), dim3(TILE), 0, s,
-                       keep_ghosts);
-    HIPCALL(hipGetLastError());
-  }
   for (int st = 1; st <= 4; ++st) {
-    const double* in = inplace ? u : ins[st - 1];
-    StageArgs a{};
-    a.r = RhsArgs{c->d_blocks, launch_of(c, BOX_INTERIOR), in, c->dv, mat, nullptr, rhs_params(p)};
-    a.un = (inplace && st > 1) ? W0 : u;
-    a.un_int = (inplace && st > 1) ? 1 : 0;
+    FusedArgs a{};
+    a.u = ins[st - 1];
+    a.mat = mat;
+    a.o = rhs_params(p);
+    a.sommerfeld = 1;
+    a.un = (!ghosts && st > 1) ? W1 : u;
+    a.un_int = !ghosts && st > 1;
     a.acc = ACC;
-    a.out = inplace ? u : outs[st - 1];
-    a.keep = (inplace && st == 1) ? W0 : nullptr;
+    a.out = outs[st - 1];
+    a.keep = (!ghosts && st == 1) ? W1 : nullptr;
     a.wa = Asub[st - 1] * dt;
     a.wb = Bw[st - 1] * dt;
     a.stage = st;
     a.cowling = p->cowling;
+    a.alg = !ghosts;
     a.eps_floor = p->eps_floor;
     a.tf_force = p->tf_force_regularization;
     a.force_reg = p->force_regularization;
-    const int g = grid_for(a.r.L.ntiles);
-    if (!p->cowling) {
-      int rc2 = launch_stencil(c, in, p, s);
-      if (rc2) return rc2;
-    }
-    {
-      PassTimer t(c, Z4C_PASS_ASSEMBLY, s);
-      if (ghosts)
-        hipLaunchKernelGGL((k_rk4_stage<true, false>), dim3(g), dim3(TILE), 0, s, a);
-      else
-        hipLaunchKernelGGL((k_rk4_stage<true, true>), dim3(g), dim3(TILE), 0, s, a);
-    }
-    HIPCALL(hipGetLastError());
+    rc = launch_fused(c, a, s);
+    if (rc) return rc;
     if (ghosts) {
       // SumBT's ghost values (u_n) into the stage state, then the ghost
       // update and AlgConstr of the whole block (z4c_rk4_stage's order)
       double* cur = a.out;
-      if (!all_ghosts && (cur != u || (inplace && st > 1))) {
-        GhostArgs gc{c->d_blocks, launch_of(c, BOX_GHOST), inplace ? W1 : u, cur, nullptr,
+      if (!all_ghosts && cur != u) {
+        GhostArgs gc{c->d_blocks, launch_of(c, BOX_GHOST), u, cur, nullptr,
                      p->eps_floor, p->tf_force_regularization, p->force_regularization};
         PassTimer t(c, Z4C_PASS_GHOSTS, s);
         hipLaunchKernelGGL(k_ghost_copy, dim3(grid_for(gc.L.ntiles)), dim3(TILE), 0, s, gc);
         HIPCALL(hipGetLastError());
       }
-      if (ghosts & 1) {
-        rc = launch_periodic(c, NVAR, cur, s);
-        if (rc) return rc;
-      } else if (ghosts & 2) {
-        rc = launch_exchange(c, NVAR, cur, s);
-        if (rc) return rc;
-      }
-      if (ghosts & 4) {
-        rc = launch_physical(c, NVAR, cur, s);
-        if (rc) return rc;
-      }
-      rc = launch_alg(c, p, cur, nullptr, 0, s);
+      rc = ghost_update(c, cur, ghosts, s);
+      if (!rc) rc = launch_alg(c, p, cur, nullptr, 0, s);
       if (rc) return rc;
-      continue;
-    }
-    if (st == 1) {
-      GhostArgs ga{c->d_blocks, launch_of(c, BOX_GHOST), u, W0, W1, p->eps_floor,
+    } else if (st == 1) {
+      GhostArgs ga{c->d_blocks, launch_of(c, BOX_GHOST), u, W0, nullptr, p->eps_floor,
                    p->tf_force_regularization, p->force_regularization};
-      {
-        PassTimer t(c, Z4C_PASS_GHOSTS, s);
-        if (inplace)
-          hipLaunchKernelGGL(k_rk4_ghosts_inplace, dim3(grid_for(ga.L.ntiles)), dim3(TILE), 0, s,
-                             ga);
-        else
-          hipLaunchKernelGGL(k_rk4_ghosts, dim3(grid_for(ga.L.ntiles)), dim3(TILE), 0, s, ga);
-      }
+      PassTimer t(c, Z4C_PASS_GHOSTS, s);
+      hipLaunchKernelGGL(k_rk4_ghosts, dim3(grid_for(ga.L.ntiles)), dim3(TILE), 0, s, ga);
       HIPCALL(hipGetLastError());
     }
   }
@@ -5041,16 +5193,6 @@ int launch_wave(z4c_ctx* c, double* out, const double* in1, const double* in2, d
   return Z4C_OK;
 }
 
-int ghost_update(z4c_ctx* c, double* u, int ghosts, hipStream_t s) {
-  int rc = Z4C_OK;
-  if (ghosts & 1)
-    rc = launch_periodic(c, NVAR, u, s);
-  else if (ghosts & 2)
-    rc = launch_exchange(c, NVAR, u, s);
-  if (!rc && (ghosts & 4)) rc = launch_physical(c, NVAR, u, s);
-  return rc;
-}
-
 int check_ls(const z4c_ls_tableau* t, bool need_2s, const char* what) {
   if (!t || t->nstages < 1 || t->nstages > Z4C_LS_MAX_STAGES)
     return fail(Z4C_EINVAL, std::string(what) + ": bad tableau");
@@ -5062,59 +5204,46 @@ int check_ls(const z4c_ls_tableau* t, bool need_2s, const char* what) {
   return Z4C_OK;
 }
 
-// Fused low-storage step.  In place (no Sommerfeld face): each stage reads
-// the state only at its own vertex, so the stage writes over the interior
-// of u; u1 lives interior-indexed in work.  With Sommerfeld faces the stage
-// reads neighbouring values of its input, so the stage states alternate
-// between u and the second work register, each stage's output first
-// receiving its input's ghosts.
+// Fused low-storage step: the stage states alternate between u and the second
+// work register (a stage reads its neighbours' vertices), each stage's output
+// first receiving its input's ghosts; u1 lives interior-indexed in work.
 int launch_ls_step(z4c_ctx* c, const z4c_params* p, const z4c_ls_tableau* T, double dt,
                    double* u, double* work, const double* mat, int ghosts, hipStream_t s) {
   const long long n = c->total_pts * NVAR;
   double* U1 = work;
   double* W = work + n;
-  bool faces = false;
-  for (const DevBlock& B : c->hdev) faces = faces || B.faces != 0;
   double* cur = u;
   int rc = Z4C_OK;
   for (int st = 1; st <= T->nstages; ++st) {
-    double* nxt = faces ? (cur == u ? W : u) : u;
-    if (faces) {
+    double* nxt = cur == u ? W : u;
+    {
       GhostArgs gc{c->d_blocks, launch_of(c, BOX_GHOST), cur, nxt, nullptr, p->eps_floor,
                    p->tf_force_regularization, p->force_regularization};
       PassTimer t(c, Z4C_PASS_GHOSTS, s);
       hipLaunchKernelGGL(k_ghost_copy, dim3(grid_for(gc.L.ntiles)), dim3(TILE), 0, s, gc);
       HIPCALL(hipGetLastError());
     }
-    StageArgs a{};
-    a.r = RhsArgs{c->d_blocks, launch_of(c, BOX_INTERIOR), cur, c->dv, mat, nullptr, rhs_params(p)};
-    a.un = cur;
+    FusedArgs a{};
+    a.u = cur;
+    a.mat = mat;
+    a.o = rhs_params(p);
+    a.sommerfeld = 1;
     a.acc = U1;
     a.out = nxt;
     a.stage = st;
     a.cowling = p->cowling;
+    a.alg = !ghosts;
     a.eps_floor = p->eps_floor;
     a.tf_force = p->tf_force_regularization;
     a.force_reg = p->force_regularization;
-    a.u1 = U1;
+    a.ls = 1;
     a.ls_w[0] = T->delta[st - 1];
     a.ls_w[1] = T->gamma_1[st - 1];
     a.ls_w[2] = T->gamma_2[st - 1];
     a.ls_w[3] = T->beta[st - 1] * dt;  // dt_scaled (time_integrators.hpp:37-40)
     a.ls_last = st == T->nstages;
-    if (!p->cowling) {
-      rc = launch_stencil(c, cur, p, s);
-      if (rc) return rc;
-    }
-    {
-      PassTimer t(c, Z4C_PASS_ASSEMBLY, s);
-      const int g = grid_for(a.r.L.ntiles);
-      if (ghosts)
-        hipLaunchKernelGGL((k_rk4_stage<true, false, true>), dim3(g), dim3(TILE), 0, s, a);
-      else
-        hipLaunchKernelGGL((k_rk4_stage<true, true, true>), dim3(g), dim3(TILE), 0, s, a);
-    }
-    HIPCALL(hipGetLastError());
+    rc = launch_fused(c, a, s);
+    if (rc) return rc;
     if (ghosts) {
       rc = ghost_update(c, nxt, ghosts, s);
       if (!rc) rc = launch_alg(c, p, nxt, nullptr, 0, s);

@@ -17,15 +17,17 @@ INCLUDE = os.path.join(ROOT, "include")
 LIB = os.path.join(PKG, "libz4c_mi355x.so")
 SOURCES = [os.path.join(CSRC, "z4c_kernels.hip")]
 HEADERS = [os.path.join(CSRC, f) for f in ("z4c_device.hpp", "z4c_rhs_point.hpp", "z4c_stencil.hpp", "z4c_adjoint.hpp",
-                                           "z4c_refine.hpp")] + [
+                                           "z4c_refine.hpp", "z4c_mesh.hpp", "z4c_fused.hpp")] + [
     os.path.join(INCLUDE, "z4c_mi355x.h")]
 
 # -ffp-contract=off: no fused multiply-add, so every product and sum rounds
 # as in the reference build (configure.py:1145) and the CPU oracle.
+# -fno-signed-zeros: a sum's leading 0 + x is dropped (the only results that
+# can differ are the signs of zeros).
 # -packed-fp32-ops off: no packed FP32 instructions anywhere in the library.
 HIPCC_FLAGS = [
     "-O3", "--offload-arch=gfx950", "-std=c++17", "-fPIC", "-shared",
-    "-ffp-contract=off",
+    "-ffp-contract=off", "-fno-signed-zeros",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-I" + INCLUDE, "-I" + CSRC,
 ]

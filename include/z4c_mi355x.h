@@ -434,17 +434,22 @@ int z4c_history_noalloc(z4c_ctx* ctx, const z4c_params* p, const double* u,
                         const double* con, double* out, void* stream);
 
 /* Tile autotuner of the stencil pass (no counterpart in the reference,
-   whose pencil loops have no tiling).  For every block size among the
+   whose pencil loops have no tiling).  Steps form their right-hand sides in
+   one kernel, and so does z4c_rhs; z4c_rhs runs a stencil pass and an algebra
+   pass for a few small blocks (at most 11 vertices along z), where that is
+   faster, for a right-hand side written over its own input, and after
+   z4c_set_stencil_threads.  For every block size among the
    registered blocks, times the stencil pass of those blocks under each
    workgroup configuration (192, 256, 320, 384, 576 or 640 threads, each with the
    fewest x-y tiles that fit) on state `u`, `reps` launches each, and keeps
    the fastest.  Until it is called a block uses 256 threads, or 192 when
    its whole x-y plane fits one 192-thread tile.  Results do not depend on
-   the configuration.
+   the configuration.  Undoes z4c_set_stencil_threads' choice of two passes.
    Waits for the stream. */
 int z4c_autotune(z4c_ctx* ctx, const z4c_params* p, const double* u, int reps, void* stream);
 /* Workgroup size the stencil pass uses for `block`; setting it (block -1:
-   all blocks) replaces the tuned or default choice. */
+   all blocks) replaces the tuned or default choice and has z4c_rhs run in
+   two passes (its result does not change). */
 int z4c_stencil_threads(z4c_ctx* ctx, int block, int* threads);
 int z4c_set_stencil_threads(z4c_ctx* ctx, int block, int threads);
 
@@ -475,7 +480,9 @@ enum {
    timing is wall-clock per cycle, src/main.cpp).  While enabled, every pass
    launch is bracketed by HIP events on its own stream.  z4c_get_timing
    waits for the recorded events, returns the summed milliseconds and the
-   launch count per pass (arrays of npass entries) and clears the record. */
+   launch count per pass (arrays of npass entries) and clears the record.  A
+   one-kernel right-hand side counts as a launch of the stencil and of the
+   assembly pass, its time divided 57:43 as their arithmetic is. */
 int z4c_set_timing(z4c_ctx* ctx, int enable);
 int z4c_get_timing(z4c_ctx* ctx, double* ms_total, long long* launches, int npass);
 
