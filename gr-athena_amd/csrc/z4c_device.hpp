@@ -154,8 +154,9 @@ constexpr int TILE = 256;
 
 // Box kinds used by the launch tables.
 // BOX_GHOST holds six boxes per block that together cover exactly the
-// ghost vertices (the padded block minus the interior).
-enum BoxKind : int { BOX_INTERIOR = 0, BOX_PREP = 1, BOX_WHOLE = 2, BOX_GHOST = 3, NBOX = 4 };
+// ghost vertices (the padded block minus the interior).  BOX_FACE holds three
+// per block with one vertex of every set of periodic images.
+enum BoxKind : int { BOX_INTERIOR = 0, BOX_PREP = 1, BOX_WHOLE = 2, BOX_GHOST = 3, BOX_FACE = 4, NBOX = 5 };
 
 struct Box {
   int lo[3];   // i, j, k
