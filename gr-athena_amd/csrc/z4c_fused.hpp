@@ -13,11 +13,11 @@
 //
 // Against the two-pass form (stencil pass writing 106 values a vertex, algebra
 // pass reading them back: 67 GB of HBM traffic per stage of 2048 blocks of
-// 16^3 .. 32^3 cells, 17.0 ms) a stage moves 26 GB and takes 12.2 ms: of that,
-// about 7 ms are FP64 and integer issue (9000 instructions a wave, no FMA), 4 to
+// 16^3 .. 32^3 cells, 17.0 ms) a stage moves 26 GB and takes 12.0 ms: of that,
+// about 7 ms are FP64 and integer issue (8300 instructions a wave, no FMA), 4 to
 // 5 ms LDS reads (55 a vertex and field with second derivatives), which the
 // barriers between fields keep from overlapping fully.  One 32^3 block's
-// right-hand side: 79 -> 42 us.
+// right-hand side: 79 -> 40 us.
 //
 // What it takes to get there, each measured: no vector load and no spill
 // reload between the window loads and the next field (the memory counter is
@@ -45,12 +45,11 @@ struct FusedCfg {
   // field window: the brick +-4, rows padded to whole 16-byte pairs
   static constexpr int PX = (BX + 8 + 1) / 2 * 2, PY = BY + 8, PZ = BZ + 8;
   static constexpr int PLANE = PX * PY;
-  // one load instruction of a wave takes RPI rows, LPR 16-byte pairs each
-  static constexpr int LPR = PX / 2, RPI = 64 / LPR, ROWS = PY * PZ;
-  static constexpr int STEP = RPI * WAVES;                  // rows per round
-  static constexpr int ROUNDS = (ROWS + STEP - 1) / STEP;
-  static_assert(ROUNDS <= 10, "drop and wrap bits of a lane");
-  static constexpr int WIN = (ROWS + RPI - 1) / RPI * RPI * PX;  // doubles
+  // a window in 16-byte pairs, 64 a load instruction, dealt to the waves in turn
+  static constexpr int PAIRS = PLANE * PZ / 2, NLD = (PAIRS + 63) / 64;
+  static constexpr int ROUNDS = (NLD + WAVES - 1) / WAVES;
+  static_assert(ROUNDS == 8, "the offsets of a lane are two 16-byte reads");
+  static constexpr int WIN = PLANE * PZ;  // doubles
   // Dx_y on the brick +-3 in x; Dx_z on the brick +-3 in x and in y
   static constexpr int DX = BX + 6;
   static constexpr int DYP = DX * BY, DZP = DX * (BY + 6);
@@ -59,14 +58,13 @@ struct FusedCfg {
   static constexpr int HX = 6 * BY * BZ, HY = BX * 6 * BZ;
   static constexpr int SX = (HX + 63) / 64, SY = (HY + 63) / 64;  // wave slots
   static constexpr int HROUNDS = (2 * SX + SY + WAVES - 1) / WAVES;
-  static constexpr int NCOL = 4;  // per-thread LDS columns
-  static constexpr int LDS = (2 * WIN + NDY + NDZ + NCOL * TH) * 8 + (HROUNDS + 1) * TH * 4;
+  static constexpr int LDS = (2 * WIN + NDY + NDZ) * 8 + (HROUNDS + 1 + ROUNDS) * TH * 4;
   static_assert(LDS <= 80 * 1024, "two workgroups per CU");
 };
 // 17 vertices along x are a row of the 16-cell blocks most runs are made of,
 // and half of a 32-cell one.  Measured on 2048 blocks of 17^3 .. 33^3 vertices:
 // one workgroup of 512 threads per CU on 17 x 6 x 5 bricks 62.1 ms a step, two
-// of 256 on 17 x 5 x 3 52.0 (at a barrier or a load of one, the other runs).
+// of 256 on 17 x 5 x 3 51.1 (at a barrier or a load of one, the other runs).
 using FuCfg = FusedCfg<17, 5, 3, 256>;
 
 struct FusedTile {
@@ -197,9 +195,10 @@ __host__ __device__ constexpr bool fu_mixed(int f) {
   return dkind(f) == DK_FULL || dkind(f) == DK_METRIC;
 }
 
-// fields whose LD term waits in the destination (the metric and A~)
+// fields whose LD term waits in the destination until the shift's derivatives
+// are known
 __host__ __device__ constexpr bool fu_stash(int f) {
-  return (f >= V_GXX && f < V_GXX + 6) || (f >= V_AXX && f < V_AXX + 6);
+  return f != V_KHAT && f != V_THETA && f < V_ALPHA;
 }
 
 template <class C>
@@ -209,18 +208,16 @@ struct FusedPoint {
   double c1[3], c2[3], cd[3];  // stencil scalings (wave-uniform)
   double* win[2];         // field windows
   double* der;            // derived planes: Dx_y, then Dx_z
-  int wave;
-  unsigned voff0;         // byte offset of this lane's pair in the first round
-  unsigned bits;          // per round: not needed by fields with (0-9) and without
-                          // (10-19) mixed derivatives; the next round's row
-                          // lies one plane further (20-29); bit 31: no pair
-  int step0, step1;       // bytes from round to round, and in addition across a plane
+  int wave, lane;
+  const int4* offs;       // byte offsets of this lane's pairs, one a round (LDS); bit 31: no
+                          // field needs the pair, bit 30: only fields with mixed
+                          // derivatives (either is out of the field's range)
   int o;                     // this vertex in a window
   const int* halo;        // this thread's vertex in the derived planes (last entry:
                           // Dx_y's index | Dx_z's << 16) and its halo values (LDS, one a round): window index |
                           // derived-plane index << 16 (negative: none)
   unsigned p8;            // this vertex in a field, bytes (no vertex: out of range)
-  double* dst;            // destination of the block: holds the LD terms of g~ and A~
+  double* dst;            // destination of the block: holds LD terms (fu_stash)
                           // until the end
   double pend;            // LD of the field before, stored past the next barrier
   double diss, bx, by, bz;
@@ -233,24 +230,19 @@ struct FusedPoint {
     return bload(make_buf(ub + (long long)f * N, (long long)N * 8), p8, 0);
   }
 
-  // starts the loads of field f's window
+  // starts the loads of field F's window
   template <int F, int PAR>
   __device__ __forceinline__ void fetch() const {
-    // opaque copies: the offsets are formed again for every field instead of
-    // being held (and spilled) through all of them
     const Buf U = make_buf(ub + (long long)F * N, (long long)N * 8);
-    unsigned v = opaque(voff0);
-    const unsigned bits = opaque(this->bits);
-    if ((int)bits < 0) return;  // past the rows of an instruction
+    const int4 a = offs[0], b = offs[C::THREADS];
+    const int v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
     for (int r = 0; r < C::ROUNDS; ++r) {
-      const int row = (r * C::WAVES + wave) * C::RPI;
-      if ((r + 1) * C::STEP <= C::ROWS || row < C::ROWS) {
-        const unsigned drop = ((bits >> (fu_mixed(F) ? r : 10 + r)) & 1u) << 31;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(U.r, (lds_ptr)(win[PAR] + row * C::PX), 16,
-                                                 v | drop, 0, 0, 0);
-      }
-      v += step0 + (-(int)((bits >> (20 + r)) & 1u) & step1);
+      const int q = r * C::WAVES + wave;
+      // every lane writes LDS, needed or not: none may past the window
+      if ((r + 1) * C::WAVES * 64 <= C::PAIRS || q * 64 + lane < C::PAIRS)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(U.r, (lds_ptr)(win[PAR] + q * 128), 16,
+                                                 fu_mixed(F) ? v[r] & ~(1 << 30) : v[r], 0, 0, 0);
     }
   }
 
@@ -327,14 +319,13 @@ struct FusedPoint {
   }
 };
 
-// The right-hand side of one vertex: fields in fu_field's order, each
-// term in the reference's operation order (z4c_rhs_point.hpp's).  k(n, value)
-// receives the 22 values; `col(c)` is this thread's LDS column c.
-template <class C, class Col>
+// The right-hand side of one vertex into k: fields in fu_field's order, each
+// term in the reference's operation order (z4c_rhs_point.hpp's).
+template <class C>
 __device__ __forceinline__ void fused_rhs(FusedPoint<C>& P, const KernArgs<FusedArgs>& ka,
-                                          const double* mat, Col&& col,
-                                          double& kK, double& kT, double& kal, double* kb,
-                                          double* kg, double* kA) {
+                                          const double* mat, double (&k)[NVAR]) {
+  double &kchi = k[V_CHI], &kK = k[V_KHAT], &kT = k[V_THETA], &kal = k[V_ALPHA];
+  double *kg = k + V_GXX, *kA = k + V_AXX, *kG = k + V_GAMX, *kb = k + V_BETAX;
   auto m = [&](int f) {
     return bload(make_buf(mat + (long long)f * P.N, (long long)P.N * 8), P.p8, 0);
   };
@@ -352,7 +343,8 @@ __device__ __forceinline__ void fused_rhs(FusedPoint<C>& P, const KernArgs<Fused
 #define Z4C_GAM(c)                                     \
   P.template field<c>(dGam[c], dd, L, D);              \
   pin(dGam[c]);                                        \
-  col(c) = L + D;
+  P.pend = L + D;                                      \
+  pin(P.pend);
   Z4C_GAM(0) Z4C_GAM(1) Z4C_GAM(2)
 #undef Z4C_GAM
   // -------------------------------------------------------------- metric
@@ -444,7 +436,8 @@ __device__ __forceinline__ void fused_rhs(FusedPoint<C>& P, const KernArgs<Fused
   // ----------------------------------------- conformal factor (:402-458)
   double dchi[3], dphi[3];
   const double chi = P.template field<9>(dchi, dd, L, D);
-  col(3) = L + D;
+  P.pend = L + D;
+  pin(P.pend);
   double oochi;
   {
   const auto& o = ka.get().o;
@@ -652,9 +645,9 @@ __device__ __forceinline__ void fused_rhs(FusedPoint<C>& P, const KernArgs<Fused
   }
   {
     const double K = P.at(V_KHAT) + 2. * P.at(V_THETA);
-    double Lchi = col(3);
+    double Lchi = P.stashed(V_CHI);
     Lchi += (1. / 6.) * pw * chi_guarded * dbeta_div;
-    col(3) = Lchi - (1. / 6.) * pw * chi_guarded * alpha * K;
+    kchi = Lchi - (1. / 6.) * pw * chi_guarded * alpha * K;
   }
   const double oopsi4 = (pw == -4.) ? chi_guarded : pow(chi_guarded, -4. / pw);
   double Str = 0.0;
@@ -681,7 +674,7 @@ __device__ __forceinline__ void fused_rhs(FusedPoint<C>& P, const KernArgs<Fused
     }
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      double LGam = col(a);
+      double LGam = P.stashed(V_GAMX + a);
       LGam += (2. / 3.) * Gu[a] * dbeta_div;
 #pragma unroll
       for (int b = 0; b < 3; ++b) {
@@ -697,7 +690,7 @@ __device__ __forceinline__ void fused_rhs(FusedPoint<C>& P, const KernArgs<Fused
         t -= 2. * Auu[sym(a, b)] * dalpha[b];
         if (mat) t -= 16. * M_PI * alpha * guu[sym(a, b)] * m(M_SX + b);
       }
-      col(a) = t;
+      kG[a] = t;
     }
   }
   __builtin_amdgcn_sched_barrier(0);

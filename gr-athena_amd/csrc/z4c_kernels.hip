@@ -414,15 +414,14 @@ k_fused(FusedArgs args) {
   __shared__ __align__(16) double winA[C::WIN];
   __shared__ __align__(16) double winB[C::WIN];
   __shared__ double der[C::NDY + C::NDZ];
-  __shared__ double cols[C::NCOL * C::THREADS];
+  __shared__ int4 offs[2 * C::THREADS];
   __shared__ int halo[(C::HROUNDS + 1) * C::THREADS];
   const KernArgs<FusedArgs> ka;
   const int G = gridDim.x;  // multiple of 8: XCD-contiguous ranges
   const int t = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
   if (t >= args.ntiles) return;
   const int tid = threadIdx.x;
-  auto col = [&](int c) -> double& { return cols[c * C::THREADS + tid]; };
-  double kK = 0.0, kT = 0.0, kal = 0.0, kb[3] = {}, kg[6] = {}, kA[6] = {};
+  double kv[NVAR] = {};
   {
     const auto& a = args;
     const FusedTile T = a.tiles[t];
@@ -448,32 +447,32 @@ k_fused(FusedArgs args) {
     P.der = der;
     P.halo = halo + tid;
     P.wave = wave;
+    P.lane = lane;
     {
-      const int row0 = wave * C::RPI + lane / C::LPR, c0 = 2 * (lane % C::LPR);
-      int kk = row0 / C::PY, jj = row0 - kk * C::PY;
-      P.step0 = 8 * B.nn1 * (C::STEP / C::PY * B.nn2 + C::STEP % C::PY);
-      P.step1 = 8 * B.nn1 * (B.nn2 - C::PY);
-      P.voff0 = 8u * (unsigned)((B.il + T.i0 - 4 + c0) +
-                                B.nn1 * ((B.jl + T.j0 - 4 + jj) + B.nn2 * (B.kl + T.k0 - 4 + kk)));
-      P.bits = lane >= C::LPR * C::RPI ? 1u << 31 : 0u;
-      // the pair's nearest distance from the brick along x
-      const int dx = c0 + 1 < 4 ? 3 - c0 : max(0, c0 - T.ni - 3);
+      int v[C::ROUNDS];
 #pragma unroll
       for (int r = 0; r < C::ROUNDS; ++r) {
-        // the row's distances in y and z; a field needs the vertices that lie
-        // off the brick along one axis (by up to 4) and, with mixed
-        // derivatives, along two (by up to 3)
+        const int e = (r * C::WAVES + wave) * 64 + lane;
+        const int row = e / (C::PX / 2), c0 = 2 * (e - row * (C::PX / 2));
+        const int kk = row / C::PY, jj = row - kk * C::PY;
+        // the pair's distances from the brick: a field needs the vertices that
+        // lie off it along one axis (by up to 4) and, with mixed derivatives,
+        // along two (by up to 3)
+        const int dx = c0 + 1 < 4 ? 3 - c0 : max(0, c0 - T.ni - 3);
         const int dy = jj < 4 ? 4 - jj : max(0, jj - T.nj - 3);
         const int dz = kk < 4 ? 4 - kk : max(0, kk - T.nk - 3);
         const int off = (dx > 0) + (dy > 0) + (dz > 0);
         const int far = max(dx, max(dy, dz));
         const bool star = off <= 1 && far <= 4;
         const bool need = star || (off == 2 && far <= 3);
-        const bool wrap = jj + C::STEP % C::PY >= C::PY;
-        P.bits |= (need ? 0u : 1u << r) | (star ? 0u : 1u << (10 + r)) | (wrap ? 1u << (20 + r) : 0u);
-        jj += C::STEP % C::PY - (wrap ? C::PY : 0);
-        kk += C::STEP / C::PY + (wrap ? 1 : 0);
+        v[r] = 8 * ((B.il + T.i0 - 4 + c0) +
+                    B.nn1 * ((B.jl + T.j0 - 4 + jj) + B.nn2 * (B.kl + T.k0 - 4 + kk)));
+        if (!need || e >= C::PAIRS) v[r] = (int)DV_DROP;
+        else if (!star) v[r] |= 1 << 30;
       }
+      offs[tid] = int4{v[0], v[1], v[2], v[3]};
+      offs[C::THREADS + tid] = int4{v[4], v[5], v[6], v[7]};
+      P.offs = offs + tid;
     }
     P.o = (tx + 4) + C::PX * (ty + 4) + C::PLANE * (tz + 4);
     halo[C::HROUNDS * C::THREADS + tid] =
@@ -514,11 +513,7 @@ k_fused(FusedArgs args) {
     P.bz = P.at(V_BETAX + 2);
     if (!a.cowling) P.template fetch<fu_field(0), 0>();
     if (!a.cowling) {
-      fused_rhs<C>(P, ka, a.mat ? a.mat + B.off * NMAT : nullptr, col, kK, kT, kal, kb,
-                   kg, kA);
-    } else {
-#pragma unroll
-      for (int c = 0; c < C::NCOL; ++c) col(c) = 0.0;
+      fused_rhs<C>(P, ka, a.mat ? a.mat + B.off * NMAT : nullptr, kv);
     }
   }
   // the tile again (nothing of it is held through the fields)
@@ -534,25 +529,15 @@ k_fused(FusedArgs args) {
   const int p = flat(B, i, j, k);
   const long long base = B.off * NVAR;
   const double* u = a.u + base + p;
-  auto kv = [&](int n) -> double& {
-    if (n == V_CHI) return col(3);
-    if (n >= V_GXX && n < V_GXX + 6) return kg[n - V_GXX];
-    if (n == V_KHAT) return kK;
-    if (n >= V_AXX && n < V_AXX + 6) return kA[n - V_AXX];
-    if (n >= V_GAMX && n < V_GAMX + 3) return col(n - V_GAMX);
-    if (n == V_THETA) return kT;
-    if (n == V_ALPHA) return kal;
-    return kb[n - V_BETAX];
-  };
   if (a.sommerfeld && !a.cowling && B.faces && on_sommerfeld_face(B, i, j, k)) {
     const Pt P = make_pt(p, B.nn1, B.nn2, N);
     sommerfeld_point(B, make_buf(a.u + base, (long long)NVAR * N * 8), P, a.u + base, i, j, k, N,
-                     [&](int n, double v) { kv(n) = v; });
+                     [&](int n, double v) { kv[n] = v; });
   }
   if (a.rhs) {
     double* rhs = a.rhs + base + p;
 #pragma unroll
-    for (int n = 0; n < NVAR; ++n) rhs[(long long)n * N] = kv(n);
+    for (int n = 0; n < NVAR; ++n) rhs[(long long)n * N] = kv[n];
     return;
   }
   const int qi = (i - B.il) + B.ni * ((j - B.jl) + B.nj * (k - B.kl));
@@ -578,7 +563,7 @@ k_fused(FusedArgs args) {
         v = (g2 == 1.0) ? v1 : g2 * v1;
       else
         v = (g2 != 0.0) ? g1 * u0 + g2 * v1 : u0 * g1;
-      s[n] = v + bdt * kv(n);
+      s[n] = v + bdt * kv[n];
     }
   } else {
     const double wa = a.wa, wb = a.wb;
@@ -597,7 +582,7 @@ k_fused(FusedArgs args) {
     }
 #pragma unroll
     for (int n = 0; n < NVAR; ++n) {
-      const double v = kv(n);
+      const double v = kv[n];
       if (stage == 1) {
         if (keep) st_state(keep + (long long)n * NI, s[n]);
         st_state(acc + (long long)n * NI, s[n] + wb * v);
