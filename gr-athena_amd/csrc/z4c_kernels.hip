@@ -950,7 +950,8 @@ struct ConArgs {
   double chi_psi_power, chi_div_floor, r_max_con;
 };
 
-__global__ void __launch_bounds__(TILE) k_constraints(ConArgs a) {
+__global__ void __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(2)))
+k_constraints(ConArgs a) {
   int b, i, j, k;
   if (!tile_point(a.L, b, i, j, k)) return;
   const DevBlock B = a.blocks[b];
@@ -2430,7 +2431,8 @@ struct AdjArgs {
 };
 
 
-__global__ void __launch_bounds__(TILE) k_adj_fwd(AdjArgs a) {
+__global__ void __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(2)))
+k_adj_fwd(AdjArgs a) {
   int b, i, j, k;
   if (!tile_point(a.L, b, i, j, k)) return;
   const DevBlock B = a.blocks[b];
