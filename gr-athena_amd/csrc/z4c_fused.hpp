@@ -13,18 +13,19 @@
 //
 // Against the two-pass form (stencil pass writing 106 values a vertex, algebra
 // pass reading them back: 67 GB of HBM traffic per stage of 2048 blocks of
-// 16^3 .. 32^3 cells, 17.0 ms) a stage moves 26 GB and takes 12.0 ms: of that,
-// about 7 ms are FP64 and integer issue (8300 instructions a wave, no FMA), 4 to
-// 5 ms LDS reads (55 a vertex and field with second derivatives), which the
+// 16^3 .. 32^3 cells, 17.0 ms) a stage moves 37 GB (25.4 read, 11.5 written:
+// the windows' halos come mostly from L2) and takes 11.4 ms.  Of that, 5.5 ms
+// are FP64 and integer issue (8000 instructions a wave, no FMA) and 4 to 5 ms
+// LDS reads (55 a vertex and field with second derivatives), which the
 // barriers between fields keep from overlapping fully.  One 32^3 block's
 // right-hand side: 79 -> 40 us.
 //
 // What it takes to get there, each measured: no vector load and no spill
 // reload between the window loads and the next field (the memory counter is
-// in order, so either waits for the whole window: 82 and 62 ms a step); the
-// offsets formed anew from two registers for every field; barriers that wait
-// for LDS traffic only; every load of the update issued before its first
-// store (68 -> 60 ms).
+// in order, so either waits for the whole window: 82 and 62 ms a step); a
+// lane's window offsets kept in LDS, not formed anew for every field (52.1 ->
+// 51.1 ms a step); barriers that wait for LDS traffic only; every load of the
+// update issued before its first store (68 -> 60 ms).
 //
 // The operation order is the two-pass form's throughout
 // (z4c_rhs_point.hpp, z4c_stencil.hpp): results are equal bit for bit.

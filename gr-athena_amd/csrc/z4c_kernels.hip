@@ -604,16 +604,14 @@ k_fused(FusedArgs args) {
 // Ghost vertices of a fused step with ghosts held at u_n: what the unfused
 // sequence leaves there after every stage is AlgConstr(u_n + 0), so the step
 // applies AlgConstr to the state's ghosts once (after the first stage has
-// read them).  The in-place step keeps every stage state in the caller's
-// state, whose ghosts are then the only copy; the step with separate stage
-// registers (Sommerfeld faces read neighbouring stage values, so the stage
-// cannot overwrite its input) also copies them into the two registers.
+// read them), and copies them into the work register that the stages alternate
+// with.  The 30.3 M ghost vertices of 2048 blocks of 16^3 .. 32^3 cells: 18.8 GB
+// (8.9 read, 9.9 written; ghost rows of 32 bytes) in 2.9 to 5.4 ms a step.
 struct GhostArgs {
   const DevBlock* blocks;
   Launch L;
   double* u;
   double* w0;
-  double* w1;
   double eps_floor;
   int tf_force, force_reg;
 };
@@ -950,6 +948,8 @@ struct ConArgs {
   double chi_psi_power, chi_div_floor, r_max_con;
 };
 
+// Two waves a SIMD although 67 registers spill (328 unbounded, one wave): the
+// loads' latency costs more, 2.03 -> 1.92 ms for 400 uneven blocks.
 __global__ void __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(2)))
 k_constraints(ConArgs a) {
   int b, i, j, k;
@@ -2430,7 +2430,8 @@ struct AdjArgs {
   long long creg;    // (NCARRY + 18) * total_int
 };
 
-
+// Two waves a SIMD, no spill (336 registers and one wave unbounded): 0.74 ->
+// 0.56 ms for 320 blocks of 16^3.
 __global__ void __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(2)))
 k_adj_fwd(AdjArgs a) {
   int b, i, j, k;
@@ -3273,7 +3274,12 @@ void launch_stencil_cfg(int cfg, const StencilArgs& sa, hipStream_t s) {
 // The derivative slots, allocated by the first two-pass right-hand side.
 int ensure_slots(z4c_ctx* c) {
   if (c->dv) return Z4C_OK;
-  if (hipMalloc(&c->dv, sizeof(double) * c->total_dv) != hipSuccess) {
+  // also while the caller captures a graph: the allocation is no part of it
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  HIPCALL(hipThreadExchangeStreamCaptureMode(&mode));
+  const hipError_t e = hipMalloc(&c->dv, sizeof(double) * c->total_dv);
+  HIPCALL(hipThreadExchangeStreamCaptureMode(&mode));
+  if (e != hipSuccess) {
     c->dv = nullptr;
     return fail(Z4C_ENOMEM, "derivative-slot allocation failed");
   }
@@ -5266,7 +5272,7 @@ int launch_rk4_step(z4c_ctx* c, const z4c_params* p, double dt, double* u, doubl
       // update and AlgConstr of the whole block (z4c_rk4_stage's order)
       double* cur = a.out;
       if (!all_ghosts && cur != u) {
-        GhostArgs gc{c->d_blocks, launch_of(c, BOX_GHOST), u, cur, nullptr,
+        GhostArgs gc{c->d_blocks, launch_of(c, BOX_GHOST), u, cur,
                      p->eps_floor, p->tf_force_regularization, p->force_regularization};
         PassTimer t(c, Z4C_PASS_GHOSTS, s);
         hipLaunchKernelGGL(k_ghost_copy, dim3(grid_for(gc.L.ntiles)), dim3(TILE), 0, s, gc);
@@ -5276,7 +5282,7 @@ int launch_rk4_step(z4c_ctx* c, const z4c_params* p, double dt, double* u, doubl
       if (!rc) rc = launch_alg(c, p, cur, nullptr, 0, s);
       if (rc) return rc;
     } else if (st == 1) {
-      GhostArgs ga{c->d_blocks, launch_of(c, BOX_GHOST), u, W0, nullptr, p->eps_floor,
+      GhostArgs ga{c->d_blocks, launch_of(c, BOX_GHOST), u, W0, p->eps_floor,
                    p->tf_force_regularization, p->force_regularization};
       PassTimer t(c, Z4C_PASS_GHOSTS, s);
       hipLaunchKernelGGL(k_rk4_ghosts, dim3(grid_for(ga.L.ntiles)), dim3(TILE), 0, s, ga);
@@ -5318,7 +5324,7 @@ int launch_ls_step(z4c_ctx* c, const z4c_params* p, const z4c_ls_tableau* T, dou
   for (int st = 1; st <= T->nstages; ++st) {
     double* nxt = cur == u ? W : u;
     {
-      GhostArgs gc{c->d_blocks, launch_of(c, BOX_GHOST), cur, nxt, nullptr, p->eps_floor,
+      GhostArgs gc{c->d_blocks, launch_of(c, BOX_GHOST), cur, nxt, p->eps_floor,
                    p->tf_force_regularization, p->force_regularization};
       PassTimer t(c, Z4C_PASS_GHOSTS, s);
       hipLaunchKernelGGL(k_ghost_copy, dim3(grid_for(gc.L.ntiles)), dim3(TILE), 0, s, gc);
@@ -5352,7 +5358,7 @@ int launch_ls_step(z4c_ctx* c, const z4c_params* p, const z4c_ls_tableau* T, dou
     } else {
       // the update leaves ghosts alone; AlgConstr of the whole block
       // reaches them after every stage
-      GhostArgs ga{c->d_blocks, launch_of(c, BOX_GHOST), nxt, nullptr, nullptr, p->eps_floor,
+      GhostArgs ga{c->d_blocks, launch_of(c, BOX_GHOST), nxt, nullptr, p->eps_floor,
                    p->tf_force_regularization, p->force_regularization};
       PassTimer t(c, Z4C_PASS_GHOSTS, s);
       hipLaunchKernelGGL(k_rk4_ghosts_inplace, dim3(grid_for(ga.L.ntiles)), dim3(TILE), 0, s,

@@ -55,6 +55,27 @@ def test_one_kernel_equals_two_passes(params, matter):
     z.close()
 
 
+def test_two_passes_captured_by_a_new_context():
+    """A graph captured around the first right-hand side that needs the
+    derivative slots: written over its own input."""
+    gs = _batch()
+    z = Z4c(gs, Params(diss=0.02))
+    u = z.upload([perturbed_flat(g, seed=b) for b, g in enumerate(gs)])
+    want = u.clone()
+    z.Z4cRHS(u, None, want)
+    v = u.clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        z.Z4cRHS(v, None, v)
+    for _ in range(3):
+        v.copy_(u)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(v, want)
+    z.close()
+
+
 def test_small_batch_rule_does_not_change_results():
     """Few small blocks take the two passes, the same blocks among many the
     one kernel."""
