@@ -2839,7 +2839,7 @@ struct z4c_ctx {
   int fu_ntiles = 0;
   bool small = false;       // too little work to fill the chip with bricks (launch_rhs)
   bool per_snap = false;    // the periodic fill reads a snapshot (a block under 4 cells)
-  bool two_pass = false;    // z4c_rhs in two passes (a stencil workgroup size was fixed)
+  int form = Z4C_FORM_AUTO; // z4c_set_rhs_form
   double* snap = nullptr;  // periodic-fill snapshot / exchange scratch (lazy)
   long long snap_elems = 0;
   double* hst = nullptr;   // history partial sums (lazy)
@@ -3057,7 +3057,7 @@ struct z4c_ctx {
     hipFree(fu_tiles);
     fu_tiles = nullptr;
     fu_ntiles = 0;
-    two_pass = false;
+    form = Z4C_FORM_AUTO;
     hipFree(snap);
     hipFree(hst);
     hst = nullptr;
@@ -3271,6 +3271,11 @@ void launch_stencil_cfg(int cfg, const StencilArgs& sa, hipStream_t s) {
   }
 }
 
+// Whether z4c_rhs runs in two passes.
+bool rhs_two(const z4c_ctx* c) {
+  return c->form ? c->form == Z4C_FORM_TWO_PASSES : c->small;
+}
+
 // The derivative slots, allocated by the first two-pass right-hand side.
 int ensure_slots(z4c_ctx* c) {
   if (c->dv) return Z4C_OK;
@@ -3350,11 +3355,11 @@ int launch_stencil(z4c_ctx* c, const double* u, const z4c_params* p, hipStream_t
 int launch_rhs(z4c_ctx* c, const z4c_params* p, const double* u,
                const double* mat, double* rhs, bool sommerfeld, hipStream_t s) {
   if (p->cowling) return fill(c, rhs, 0.0, c->total_pts * NVAR, s);
-  // one kernel, unless the batch is small or the right-hand side is written
-  // over its own input (every brick reads its neighbours' vertices)
+  // one kernel, unless the batch is better off in two passes or the right-hand
+  // side is written over its own input (every brick reads its neighbours' vertices)
   const long long nn = c->total_pts * NVAR;
   const bool apart = (uintptr_t)rhs + 8 * nn <= (uintptr_t)u || (uintptr_t)u + 8 * nn <= (uintptr_t)rhs;
-  if (apart && !c->two_pass && !c->small) {
+  if (apart && !rhs_two(c)) {
     FusedArgs a{};
     a.u = u;
     a.mat = mat;
@@ -5093,9 +5098,9 @@ int z4c_autotune(z4c_ctx* c, const z4c_params* p, const double* u, int reps, voi
   int rc = check_ctx(c);
   if (rc) return rc;
   if (!p || !u || reps < 1) return fail(Z4C_EINVAL, "autotune: bad argument");
+  const bool had_slots = c->dv != nullptr;
   rc = ensure_slots(c);
   if (rc) return rc;
-  c->two_pass = false;
   hipStream_t s = (hipStream_t)stream;
   std::map<std::array<int, 3>, std::vector<int>> classes;
   for (int b = 0; b < c->nblocks; ++b)
@@ -5148,6 +5153,10 @@ int z4c_autotune(z4c_ctx* c, const z4c_params* p, const double* u, int reps, voi
   hipFree(d);
   hipEventDestroy(e0);
   hipEventDestroy(e1);
+  if (!had_slots) {  // no right-hand side of the context needed them so far
+    hipFree(c->dv);
+    c->dv = nullptr;
+  }
   if (rc) return rc;
   return build_stencil_plan(c, c->hdev);
 }
@@ -5166,8 +5175,30 @@ int z4c_set_stencil_threads(z4c_ctx* c, int block, int threads) {
       return fail(Z4C_EINVAL, "set_stencil_threads: no tile of that size fits block " +
                                   std::to_string(b));
   for (int b = b0; b < b1; ++b) c->blk_cfg[b] = q;
-  c->two_pass = true;
   return build_stencil_plan(c, c->hdev);
+}
+
+int z4c_set_rhs_form(z4c_ctx* c, int form) {
+  int rc = check_ctx(c);
+  if (rc) return rc;
+  if (form < Z4C_FORM_AUTO || form > Z4C_FORM_TWO_PASSES)
+    return fail(Z4C_EINVAL, "set_rhs_form: unknown form");
+  if (form == Z4C_FORM_TWO_PASSES) {
+    rc = ensure_slots(c);
+    if (rc) return rc;
+  }
+  c->invalidate_graph();
+  c->form = form;
+  return Z4C_OK;
+}
+
+int z4c_rhs_form(z4c_ctx* c, int* rhs, int* step) {
+  int rc = check_ctx(c);
+  if (rc) return rc;
+  if (!rhs || !step) return fail(Z4C_EINVAL, "rhs_form: null argument");
+  *rhs = rhs_two(c) ? Z4C_FORM_TWO_PASSES : Z4C_FORM_ONE_KERNEL;
+  *step = Z4C_FORM_ONE_KERNEL;
+  return Z4C_OK;
 }
 
 int z4c_stencil_threads(z4c_ctx* c, int block, int* threads) {

@@ -24,7 +24,8 @@ EXPORTS = [
     "z4c_adm_constraints", "z4c_bt_sum", "z4c_weighted_ave", "z4c_add_rhs",
     "z4c_new_dt", "z4c_periodic_fill", "z4c_rk4_stage", "z4c_rk4_step",
     "z4c_set_timing", "z4c_get_timing", "z4c_history", "z4c_set_exchange", "z4c_exchange",
-    "z4c_autotune", "z4c_stencil_threads", "z4c_set_stencil_threads", "z4c_rk4_step_graph",
+    "z4c_autotune", "z4c_stencil_threads", "z4c_set_stencil_threads", "z4c_set_rhs_form",
+    "z4c_rhs_form", "z4c_rk4_step_graph",
     "z4c_physical_bc", "z4c_rhs_vjp", "z4c_rk4_step_vjp", "z4c_hamiltonian_norm",
     "z4c_exchange_vjp", "z4c_rk4_step_ghosts_vjp", "z4c_physical_bc_vjp",
     "z4c_hamiltonian_norm_vjp", "z4c_weyl", "z4c_coarse_layout", "z4c_restrict",
@@ -153,6 +154,8 @@ def load(path: str | None = None):
         "z4c_autotune": [vp, pp, vp, i, vp],
         "z4c_stencil_threads": [vp, i, C.POINTER(i)],
         "z4c_set_stencil_threads": [vp, i, i],
+        "z4c_set_rhs_form": [vp, i],
+        "z4c_rhs_form": [vp, C.POINTER(i), C.POINTER(i)],
         "z4c_rk4_step_graph": [vp, pp, d, vp, vp, vp],
         "z4c_physical_bc": [vp, i, vp, vp],
         "z4c_get_timing": [vp, C.POINTER(d), C.POINTER(ll), i],

@@ -426,6 +426,20 @@ class Z4c:
             out[tuple(n + 1 for n in g.nx)] = t.value
         return out
 
+    RHS_FORMS = {"auto": 0, "one kernel": 1, "two passes": 2}
+
+    def set_rhs_form(self, form):
+        """Form of Z4cRHS and the stage calls: "auto" (the faster one for
+        the blocks), "one kernel" or "two passes"; results are the same."""
+        check(self.L.z4c_set_rhs_form(self._ctx, self.RHS_FORMS[form]), "set_rhs_form")
+
+    def rhs_form(self):
+        """(form of Z4cRHS and the stage calls, form of the fused steps)."""
+        f = (C.c_int(), C.c_int())
+        check(self.L.z4c_rhs_form(self._ctx, C.byref(f[0]), C.byref(f[1])), "rhs_form")
+        name = {v: k for k, v in self.RHS_FORMS.items()}
+        return name[f[0].value], name[f[1].value]
+
     def set_timing(self, enable=True):
         """Bracket every pass launch with HIP events on its stream."""
         check(self.L.z4c_set_timing(self._ctx, int(enable)), "set_timing")

@@ -434,22 +434,18 @@ int z4c_history_noalloc(z4c_ctx* ctx, const z4c_params* p, const double* u,
                         const double* con, double* out, void* stream);
 
 /* Tile autotuner of the stencil pass (no counterpart in the reference,
-   whose pencil loops have no tiling).  Steps form their right-hand sides in
-   one kernel, and so does z4c_rhs; z4c_rhs runs a stencil pass and an algebra
-   pass for a few small blocks (at most 11 vertices along z), where that is
-   faster, for a right-hand side written over its own input, and after
-   z4c_set_stencil_threads.  For every block size among the
+   whose pencil loops have no tiling).  Only right-hand sides formed in two
+   passes run it (z4c_set_rhs_form); which form they take does not depend on the
+   tuning.  For every block size among the
    registered blocks, times the stencil pass of those blocks under each
    workgroup configuration (192, 256, 320, 384, 576 or 640 threads, each with the
    fewest x-y tiles that fit) on state `u`, `reps` launches each, and keeps
    the fastest.  Until it is called a block uses 256 threads, or 192 when
    its whole x-y plane fits one 192-thread tile.  Results do not depend on
-   the configuration.  Undoes z4c_set_stencil_threads' choice of two passes.
-   Waits for the stream. */
+   the configuration.  Waits for the stream. */
 int z4c_autotune(z4c_ctx* ctx, const z4c_params* p, const double* u, int reps, void* stream);
 /* Workgroup size the stencil pass uses for `block`; setting it (block -1:
-   all blocks) replaces the tuned or default choice and has z4c_rhs run in
-   two passes (its result does not change). */
+   all blocks) replaces the tuned or default choice. */
 int z4c_stencil_threads(z4c_ctx* ctx, int block, int* threads);
 int z4c_set_stencil_threads(z4c_ctx* ctx, int block, int threads);
 
@@ -462,6 +458,19 @@ int z4c_set_stencil_threads(z4c_ctx* ctx, int block, int threads);
    the vertex coordinates x0 + i*dx. */
 int z4c_weyl(z4c_ctx* ctx, const z4c_params* p, const double* u, const double* adm,
              double* weyl, void* stream);
+
+/* Form of the right-hand sides (no counterpart in the reference): one kernel
+   per brick of vertices, or a stencil pass into derivative slots and an algebra
+   pass.  Results are equal bit for bit.  Z4C_FORM_AUTO (the default, restored by
+   z4c_set_blocks) takes the faster one for the registered blocks; the others
+   hold for every later z4c_rhs and stage call of the context.  Whatever the
+   form, a right-hand side written over its own input takes two passes and a
+   zero one (cowling) neither. */
+enum { Z4C_FORM_AUTO = 0, Z4C_FORM_ONE_KERNEL = 1, Z4C_FORM_TWO_PASSES = 2 };
+int z4c_set_rhs_form(z4c_ctx* ctx, int form);
+/* The forms that z4c_rhs and the stage calls, and the fused steps, now
+   take. */
+int z4c_rhs_form(z4c_ctx* ctx, int* rhs, int* step);
 
 /* Passes of the kernel timer. */
 enum {

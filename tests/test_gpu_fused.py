@@ -41,13 +41,14 @@ def test_one_kernel_equals_two_passes(params, matter):
                                  generator=gen)
     one = torch.full_like(u, 7.0)
     two = torch.full_like(u, 7.0)
+    z.set_rhs_form("one kernel")
     z.Z4cRHS(u, mat, one)
-    z.set_stencil_threads(192)
+    z.set_rhs_form("two passes")
     z.Z4cRHS(u, mat, two)
     assert torch.equal(one, two)
     # written over its own input
     v = u.clone()
-    z.autotune(u, reps=1)
+    z.set_rhs_form("one kernel")
     z.Z4cRHS(v, mat, v)
     for b in range(len(gs)):
         a, w = z.block_view(one, b, 22), z.block_view(v, b, 22)
@@ -76,6 +77,23 @@ def test_two_passes_captured_by_a_new_context():
     z.close()
 
 
+def test_stencil_threads_do_not_choose_the_form():
+    """Fixing or tuning the stencil pass's workgroups leaves the form of the
+    right-hand sides, and what it is measured on, as they were."""
+    z = Z4c([MeshBlockGeom.cube(32, 0.1, 0.3)], Params(diss=0.02))
+    u = z.upload([perturbed_flat(z.blocks[0], seed=1)])
+    assert z.rhs_form()[0] == "one kernel"
+    z.set_stencil_threads(256)
+    assert z.rhs_form()[0] == "one kernel"
+    z.set_rhs_form("two passes")
+    z.autotune(u, reps=1)
+    z.set_stencil_threads(192, block=0)
+    assert z.rhs_form()[0] == "two passes"
+    z.set_rhs_form("auto")
+    assert z.rhs_form()[0] == "one kernel"
+    z.close()
+
+
 def test_small_batch_rule_does_not_change_results():
     """Few small blocks take the two passes, the same blocks among many the
     one kernel."""
@@ -83,8 +101,9 @@ def test_small_batch_rule_does_not_change_results():
     many = g + [MeshBlockGeom.cube(16, 0.1, 2.0 * b + 3.0) for b in range(8)]
     p = Params(diss=0.02)
     out = []
-    for gs in (g, many):
+    for gs, form in ((g, "two passes"), (many, "one kernel")):
         z = Z4c(gs, p)
+        assert z.rhs_form()[0] == form
         u = z.upload([perturbed_flat(x, seed=b) for b, x in enumerate(gs)])
         r = z.zeros()
         z.Z4cRHS(u, None, r)
@@ -96,8 +115,9 @@ def test_small_batch_rule_does_not_change_results():
 @pytest.mark.parametrize("faces", [0, 63])
 @pytest.mark.parametrize("ghosts", [dict(), dict(physical=True)])
 def test_step_equals_stages(faces, ghosts):
-    """The fused step (state registers alternating) against the task list's
-    stage sequence on the same ragged blocks."""
+    """The fused step in one kernel (state registers alternating) against the
+    task list's stage sequence with its right-hand sides in two passes, on the
+    same ragged blocks."""
     if ghosts and not faces:
         pytest.skip("no face to fill")
     gs = _batch(faces)
@@ -108,7 +128,9 @@ def test_step_equals_stages(faces, ghosts):
     z.AlgConstr(a)
     z.AlgConstr(b)
     un, k = z.make_rk_registers()
+    z.set_rhs_form("two passes")
     z.rk4_step(0.004, a, un, k, **ghosts)
+    z.set_rhs_form("one kernel")
     z.rk4_step_fused(0.004, b, z.make_step_work(), **ghosts)
     for q in range(len(gs)):
         x, y = z.block_view(a, q, 22), z.block_view(b, q, 22)

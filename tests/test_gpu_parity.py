@@ -117,9 +117,8 @@ def test_rhs_with_matter_sources():
 
 @pytest.mark.parametrize("faces", [True, False])
 def test_fused_step_with_matter_equals_stage_sequence(faces):
-    """The fused step (in place without Sommerfeld faces, through the stage
-    registers with them) with matter sources against the stage sequence, and
-    the graph-replayed step refuses matter."""
+    """The fused step with matter sources against the stage sequence, and the
+    graph-replayed step refuses matter."""
     gs = _uneven_batch(faces)
     p = Params(**MP_GAUGE)
     host = [constrained_state(g, p, seed=80 + b) for b, g in enumerate(gs)]

@@ -39,6 +39,7 @@ def test_stencil_configurations_agree_and_autotune():
     z = Z4c(gs, p)
     u = z.upload([perturbed_flat(g, seed=3 + b) for b, g in enumerate(gs)])
     outs = []
+    z.set_rhs_form("two passes")
     for th in (192, 256, 320, 384, 576, 640):
         z.set_stencil_threads(th)
         assert set(z.stencil_plan().values()) == {th}
