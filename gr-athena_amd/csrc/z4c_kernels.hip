@@ -392,22 +392,94 @@ __global__ void __launch_bounds__(TILE) k_algconstr(AlgArgs a) {
 // pass reads them back from HBM in any case.
 __device__ __forceinline__ void st_state(double* p, double v) { __builtin_nontemporal_store(v, p); }
 
-// Right-hand side of a brick (z4c_fused.hpp), stored as such or taken into the
-// stage update.  The reference runs CalculateZ4cRHS, IntegrateZ4c (SumBT over
-// the registers) and EnforceAlgConstr as separate tasks
+// Stage update of the vertex p (interior index qi) with right-hand side kv(n),
+// then AlgConstr of the point.  The reference runs CalculateZ4cRHS, IntegrateZ4c
+// (SumBT over the registers) and EnforceAlgConstr as separate tasks
 // (src/task_list/gr/task_list_gr_z4c.cpp:46-64); the update is pointwise, so
 // every variable's follows its right-hand side, with the same sums in the same
 // order:
 //   u_{s+1} = u_n + (A[s+1][s] dt) k_s          (the one nonzero of bt_rk4's row)
 //   acc_1 = u_n + (b_1 dt) k_1,  acc_s = acc_{s-1} + (b_s dt) k_s
 //   u_{n+1} = acc_3 + (b_4 dt) k_4 = ((u_n + b_1 dt k_1) + b_2 dt k_2) + ...
-// followed by AlgConstr of the point (src/z4c/z4c.cpp:677-991).  LS: the
+// followed by AlgConstr of the point (src/z4c/z4c.cpp:677-991).  ls: the
 // low-storage 2S stage (task_list_gr_z4c.cpp:176-193) with WeightedAve_'s case
 // split (weighted_ave.cpp:21-132):
 //   u1 = WeightedAve(u1, u, -, {1, delta, 0})   (u1 = 0 before stage 1)
 //   u  = WeightedAve(u, u1, -, {gamma_1, gamma_2, 0}) + (beta dt) rhs
 // The running sum, the kept u_n and u1 are interior-indexed (whole 128-byte
 // lines of interior points).
+template <class A, class K>
+__device__ __forceinline__ void stage_update(const A& a, bool alg, bool ls, const DevBlock& B, int p,
+                                             int qi, K&& kv) {
+  const int N = B.npts;
+  const long long ibase = B.ioff * NVAR + qi;
+  const int NI = B.nint;
+  const long long base = B.off * NVAR;
+  const double* u = a.u + base + p;
+  double* out = a.out + base + p;
+  double* acc = a.acc + ibase;
+  const int stage = a.stage;
+  // every load before the first store: one wait instead of one per field
+  double s[NVAR], x[NVAR];
+  if (ls) {
+    double* u1 = acc;
+    const double dl = a.ls_w[0], g1 = a.ls_w[1], g2 = a.ls_w[2], bdt = a.ls_w[3];
+#pragma unroll
+    for (int n = 0; n < NVAR; ++n) s[n] = u[(long long)n * N];
+#pragma unroll
+    for (int n = 0; n < NVAR; ++n) x[n] = (stage == 1) ? 0.0 : u1[(long long)n * NI];
+#pragma unroll
+    for (int n = 0; n < NVAR; ++n) {
+      const double u0 = s[n];
+      double v1 = x[n];
+      if (dl != 0.0) v1 += dl * u0;
+      if (!a.ls_last) st_state(u1 + (long long)n * NI, v1);
+      double v;
+      if (g1 == 1.0)
+        v = (g2 != 0.0) ? u0 + g2 * v1 : u0;
+      else if (g1 == 0.0)
+        v = (g2 == 1.0) ? v1 : g2 * v1;
+      else
+        v = (g2 != 0.0) ? g1 * u0 + g2 * v1 : u0 * g1;
+      s[n] = v + bdt * kv(n);
+    }
+  } else {
+    const double wa = a.wa, wb = a.wb;
+    const double* un = a.un_int ? a.un + ibase : a.un + base + p;
+    const long long un_st = a.un_int ? NI : N;
+    double* keep = a.keep ? a.keep + ibase : nullptr;
+    if (stage < 4) {
+#pragma unroll
+      for (int n = 0; n < NVAR; ++n) s[n] = un[n * un_st];
+    }
+    if (stage > 1) {
+#pragma unroll
+      for (int n = 0; n < NVAR; ++n) x[n] = acc[(long long)n * NI];
+    }
+#pragma unroll
+    for (int n = 0; n < NVAR; ++n) {
+      const double v = kv(n);
+      if (stage == 1) {
+        if (keep) st_state(keep + (long long)n * NI, s[n]);
+        st_state(acc + (long long)n * NI, s[n] + wb * v);
+        s[n] = s[n] + wa * v;
+      } else if (stage < 4) {
+        st_state(acc + (long long)n * NI, x[n] + wb * v);
+        s[n] = s[n] + wa * v;
+      } else {
+        s[n] = x[n] + wb * v;
+      }
+    }
+  }
+  if (alg)
+    algconstr_vals(s + V_GXX, s + V_AXX, s[V_CHI], s[V_ALPHA], a.eps_floor, a.tf_force,
+                   a.force_reg);
+#pragma unroll
+  for (int n = 0; n < NVAR; ++n) st_state(out + (long long)n * N, s[n]);
+}
+
+// Right-hand side of a brick (z4c_fused.hpp), stored as such or taken into the
+// stage update.
 template <class C>
 __global__ void __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(2)))
 k_fused(FusedArgs args) {
@@ -511,10 +583,8 @@ k_fused(FusedArgs args) {
     P.bx = P.at(V_BETAX);
     P.by = P.at(V_BETAX + 1);
     P.bz = P.at(V_BETAX + 2);
-    if (!a.cowling) P.template fetch<fu_field(0), 0>();
-    if (!a.cowling) {
-      fused_rhs<C>(P, ka, a.mat ? a.mat + B.off * NMAT : nullptr, kv);
-    }
+    P.template fetch<fu_field(0), 0>();
+    fused_rhs<C>(P, ka, a.mat ? a.mat + B.off * NMAT : nullptr, kv);
   }
   // the tile again (nothing of it is held through the fields)
   const auto& a = ka.get();
@@ -528,8 +598,7 @@ k_fused(FusedArgs args) {
   const int i = B.il + T.i0 + tx, j = B.jl + T.j0 + ty, k = B.kl + T.k0 + tz;
   const int p = flat(B, i, j, k);
   const long long base = B.off * NVAR;
-  const double* u = a.u + base + p;
-  if (a.sommerfeld && !a.cowling && B.faces && on_sommerfeld_face(B, i, j, k)) {
+  if (a.sommerfeld && B.faces && on_sommerfeld_face(B, i, j, k)) {
     const Pt P = make_pt(p, B.nn1, B.nn2, N);
     sommerfeld_point(B, make_buf(a.u + base, (long long)NVAR * N * 8), P, a.u + base, i, j, k, N,
                      [&](int n, double v) { kv[n] = v; });
@@ -541,66 +610,49 @@ k_fused(FusedArgs args) {
     return;
   }
   const int qi = (i - B.il) + B.ni * ((j - B.jl) + B.nj * (k - B.kl));
-  const long long ibase = B.ioff * NVAR + qi;
-  const int NI = B.nint;
-  double* out = a.out + base + p;
-  double* acc = a.acc + ibase;
-  const int stage = a.stage;
-  double s[NVAR];
-  if (a.ls) {
-    double* u1 = acc;
-    const double dl = a.ls_w[0], g1 = a.ls_w[1], g2 = a.ls_w[2], bdt = a.ls_w[3];
-#pragma unroll
-    for (int n = 0; n < NVAR; ++n) {
-      const double u0 = u[(long long)n * N];
-      double v1 = (stage == 1) ? 0.0 : u1[(long long)n * NI];
-      if (dl != 0.0) v1 += dl * u0;
-      if (!a.ls_last) st_state(u1 + (long long)n * NI, v1);
-      double v;
-      if (g1 == 1.0)
-        v = (g2 != 0.0) ? u0 + g2 * v1 : u0;
-      else if (g1 == 0.0)
-        v = (g2 == 1.0) ? v1 : g2 * v1;
-      else
-        v = (g2 != 0.0) ? g1 * u0 + g2 * v1 : u0 * g1;
-      s[n] = v + bdt * kv[n];
-    }
+  stage_update(a, a.alg, a.ls, B, p, qi, [&](int n) { return kv[n]; });
+}
+
+// The stage in two passes: after the stencil pass, the algebra of one vertex
+// per thread and its update.  Curvature part and right-hand side wait in LDS
+// columns as in k_rhs_alg.  The stage reads its input at its own vertex only
+// (but for Sommerfeld rows), so without flagged faces out may be u itself.
+// A zero right-hand side (cowling) takes this kernel without the stencil pass.
+struct StageArgs {
+  FusedArgs f;  // f.tiles unused
+  Launch L;
+  const double* dv;
+};
+
+template <bool ALG, bool LS>
+__global__ void __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(2)))
+k_rk4_stage(StageArgs a) {
+  __shared__ double ko[NVAR * TILE];  // this point's k_s, staged (see k_rhs_alg)
+  __shared__ double cvs[12 * TILE];   // this point's curvature part
+  int b, i, j, k;
+  if (!tile_point(a.L, b, i, j, k)) return;
+  const int t = threadIdx.x;
+  const DevBlock B = a.f.blocks[b];
+  const int N = B.npts;
+  const int p = flat(B, i, j, k);
+  const int qi = (i - B.il) + B.ni * ((j - B.jl) + B.nj * (k - B.kl));
+  if (a.f.cowling) {
+    for (int n = 0; n < NVAR; ++n) ko[n * TILE + t] = 0.0;
   } else {
-    const double wa = a.wa, wb = a.wb;
-    const double* un = a.un_int ? a.un + ibase : a.un + base + p;
-    const long long un_st = a.un_int ? NI : N;
-    double* keep = a.keep ? a.keep + ibase : nullptr;
-    // every load before the first store: one wait instead of one per field
-    double x[NVAR];
-    if (stage < 4) {
-#pragma unroll
-      for (int n = 0; n < NVAR; ++n) s[n] = un[n * un_st];
-    }
-    if (stage > 1) {
-#pragma unroll
-      for (int n = 0; n < NVAR; ++n) x[n] = acc[(long long)n * NI];
-    }
-#pragma unroll
-    for (int n = 0; n < NVAR; ++n) {
-      const double v = kv[n];
-      if (stage == 1) {
-        if (keep) st_state(keep + (long long)n * NI, s[n]);
-        st_state(acc + (long long)n * NI, s[n] + wb * v);
-        s[n] = s[n] + wa * v;
-      } else if (stage < 4) {
-        st_state(acc + (long long)n * NI, x[n] + wb * v);
-        s[n] = s[n] + wa * v;
-      } else {
-        s[n] = x[n] + wb * v;
-      }
+    const RhsArgs r{a.f.blocks, a.L, a.f.u, a.dv, a.f.mat, nullptr, a.f.o};
+    const PointIO X = point_io(r, B, p, qi);
+    rhs_curvature_point(a.f.o, X, [&](int n, double v) { cvs[n * TILE + t] = v; });
+    rhs_assembly_point(a.f.o, X, [&](int n) { return cvs[n * TILE + t]; },
+                       [&](int n, double v) { ko[n * TILE + t] = v; });
+    if (B.faces && on_sommerfeld_face(B, i, j, k)) {
+      const Pt P = make_pt(p, B.nn1, B.nn2, N);
+      sommerfeld_point(B, X.U, P, a.f.u + B.off * NVAR, i, j, k, N,
+                       [&](int n, double v) { ko[n * TILE + t] = v; });
     }
   }
-  if (a.alg)
-    algconstr_vals(s + V_GXX, s + V_AXX, s[V_CHI], s[V_ALPHA], a.eps_floor, a.tf_force,
-                   a.force_reg);
-#pragma unroll
-  for (int n = 0; n < NVAR; ++n) st_state(out + (long long)n * N, s[n]);
+  stage_update(a.f, ALG, LS, B, p, qi, [&](int n) { return ko[n * TILE + t]; });
 }
+
 // Ghost vertices of a fused step with ghosts held at u_n: what the unfused
 // sequence leaves there after every stage is AlgConstr(u_n + 0), so the step
 // applies AlgConstr to the state's ghosts once (after the first stage has
@@ -2837,9 +2889,10 @@ struct z4c_ctx {
   long long total_dv = 0;   // doubles of the derivative slots (dv, allocated on first use)
   FusedTile* fu_tiles = nullptr;  // bricks of the one-kernel right-hand side
   int fu_ntiles = 0;
-  bool small = false;       // too little work to fill the chip with bricks (launch_rhs)
-  bool per_snap = false;    // the periodic fill reads a snapshot (a block under 4 cells)
+  double t_one = 0, t_two = 0;  // estimated right-hand side in one kernel, in two passes (us)
   int form = Z4C_FORM_AUTO; // z4c_set_rhs_form
+  bool faces = false;       // some block has a Sommerfeld face
+  bool per_snap = false;    // the periodic fill reads a snapshot (a block under 4 cells)
   double* snap = nullptr;  // periodic-fill snapshot / exchange scratch (lazy)
   long long snap_elems = 0;
   double* hst = nullptr;   // history partial sums (lazy)
@@ -3057,6 +3110,8 @@ struct z4c_ctx {
     hipFree(fu_tiles);
     fu_tiles = nullptr;
     fu_ntiles = 0;
+    t_one = t_two = 0;
+    faces = false;
     form = Z4C_FORM_AUTO;
     hipFree(snap);
     hipFree(hst);
@@ -3271,9 +3326,14 @@ void launch_stencil_cfg(int cfg, const StencilArgs& sa, hipStream_t s) {
   }
 }
 
-// Whether z4c_rhs runs in two passes.
+// Whether z4c_rhs runs in two passes, and the stages of a step: a stage in one
+// kernel pays for the second buffer that its state goes to, about 5 % of a
+// right-hand side.
 bool rhs_two(const z4c_ctx* c) {
-  return c->form ? c->form == Z4C_FORM_TWO_PASSES : c->small;
+  return c->form ? c->form == Z4C_FORM_TWO_PASSES : c->t_one >= c->t_two;
+}
+bool step_two(const z4c_ctx* c) {
+  return c->form ? c->form == Z4C_FORM_TWO_PASSES : c->t_one >= 0.95 * c->t_two;
 }
 
 // The derivative slots, allocated by the first two-pass right-hand side.
@@ -3291,14 +3351,30 @@ int ensure_slots(z4c_ctx* c) {
   return Z4C_OK;
 }
 
-// Bricks of the one-kernel right-hand side, cut as equal as they divide.
+// Bricks of the one-kernel right-hand side, cut as equal as they divide, and the
+// time of both forms.
+//
+// One kernel: a brick takes 35 to 37 us however few there are (its 22 fields in
+// turn), 53 us with a second one on its CU, 84 us when a third round begins, and
+// from there 0.0955 us a brick.  Two passes: a workgroup of the stencil pass
+// marches the planes of a tile, 1.75 us each on top of 20 us (16 us once there
+// are enough for the fields of a tile to meet on one XCD); a full chip takes
+// 0.003 us a workgroup and 0.003 us a plane, the algebra 0.1 us per 256 vertices.
+// Tiles that split a block's rows take half as long again a plane.  Against 132
+// batches measured in both forms (2 to 64 cells a side; cubes, rods, plates and
+// mixtures; 1 to 2048 blocks) the first estimate is within 5 % (rms) and the
+// second within 9 % (7 % where the two are close).  z4c_rhs in the form that they
+// favour loses 0.3 % to the better one on average and 11 % at most (64 blocks of
+// 2^3 cells, 38.0 against 34.0 us); always one kernel loses 4.4 % on average and
+// up to 58 % (16 blocks of 2^3: 34.0 against 21.5 us; 64 of 4 x 64 x 4: 160
+// against 105).
 int build_fused_tiles(z4c_ctx* c, const std::vector<DevBlock>& hb) {
   constexpr int M[3] = {FuCfg::BX, FuCfg::BY, FuCfg::BZ};
   std::vector<FusedTile> t;
-  int planes = 0;
+  double planes = 0, march = 0, wgs = 0, alg = 0;
+  std::vector<PlaneTile> pt;
   for (int b = 0; b < (int)hb.size(); ++b) {
     const int n[3] = {hb[b].ni, hb[b].nj, hb[b].nk};
-    planes = std::max(planes, n[2]);
     int s[3];
     for (int d = 0; d < 3; ++d) {
       const int q = (n[d] + M[d] - 1) / M[d];
@@ -3309,18 +3385,24 @@ int build_fused_tiles(z4c_ctx* c, const std::vector<DevBlock>& hb) {
         for (int i0 = 0; i0 < n[0]; i0 += s[0])
           t.push_back(FusedTile{b, i0, j0, k0, std::min(s[0], n[0] - i0), std::min(s[1], n[1] - j0),
                                 std::min(s[2], n[2] - k0)});
+    pt.clear();
+    plane_tiles(c->blk_cfg[b], b, n[0], n[1], &pt);
+    const double w = (double)pt.size() * NVAR;
+    wgs += w;
+    march += w * n[2] * (pt[0].ni < n[0] ? 1.5 : 1.0);
+    planes = std::max(planes, (double)n[2]);
+    alg += (hb[b].nint + TILE - 1) / TILE;
   }
   if (hipMalloc(&c->fu_tiles, sizeof(FusedTile) * t.size()) != hipSuccess)
     return fail(Z4C_ENOMEM, "set_blocks: brick table allocation failed");
   HIPCALL(hipMemcpy(c->fu_tiles, t.data(), sizeof(FusedTile) * t.size(), hipMemcpyHostToDevice));
   c->fu_ntiles = (int)t.size();
-  // The one-kernel form runs a brick's 22 fields in turn (37 us however few
-  // the bricks); the two passes split a block by field as well and march its
-  // planes.  Measured on one block: 31.7 / 34.5 / 38.0 / 41.5 us in two passes
-  // for 7 / 9 / 11 / 13 vertices a side against 37-39 us, and 30.7 against 37.3
-  // us for 16 blocks of 9^3 (96 bricks), 71.7 against 53.7 us for 64 (384).
-  c->small = t.size() <= 128 && planes <= 10;
-  return c->small ? ensure_slots(c) : Z4C_OK;
+  const double nt = (double)t.size(), cu = c->n_cu;
+  c->t_one = std::max(nt > 2 * cu ? 84.0 : nt > cu ? 53.0 : 37.0, 0.0955 * nt + 8.0);
+  const double lat = 20.0 + 1.75 * planes - (wgs >= 8 * NVAR ? 4.0 : 0.0);
+  const double thr = 12.0 + 0.003 * wgs + 0.003 * march + 0.1 * alg;
+  c->t_two = std::sqrt(std::sqrt(lat * lat * lat * lat + thr * thr * thr * thr));
+  return rhs_two(c) || step_two(c) ? ensure_slots(c) : Z4C_OK;
 }
 
 // The launch does the work of the stencil and the assembly passes: the kernel
@@ -3349,6 +3431,25 @@ int launch_stencil(z4c_ctx* c, const double* u, const z4c_params* p, hipStream_t
     launch_stencil_cfg(q, sa, s);
     HIPCALL(hipGetLastError());
   }
+  return Z4C_OK;
+}
+
+// One stage of a step: right-hand side of a.u, update and AlgConstr into a.out,
+// in one kernel or in two passes.  A zero right-hand side (cowling) always takes
+// the second pass alone.
+int launch_stage(z4c_ctx* c, const z4c_params* p, bool two, FusedArgs a, hipStream_t s) {
+  if (!two) return launch_fused(c, a, s);
+  if (!a.cowling) {
+    const int rc = launch_stencil(c, a.u, p, s);
+    if (rc) return rc;
+  }
+  a.blocks = c->d_blocks;
+  const StageArgs sa{a, launch_of(c, BOX_INTERIOR), c->dv};
+  PassTimer t(c, Z4C_PASS_ASSEMBLY, s);
+  auto* k = a.ls ? (a.alg ? k_rk4_stage<true, true> : k_rk4_stage<false, true>)
+                 : (a.alg ? k_rk4_stage<true, false> : k_rk4_stage<false, false>);
+  hipLaunchKernelGGL(k, dim3(grid_for(sa.L.ntiles)), dim3(TILE), 0, s, sa);
+  HIPCALL(hipGetLastError());
   return Z4C_OK;
 }
 
@@ -4151,7 +4252,7 @@ int z4c_set_blocks(z4c_ctx* c, const z4c_block* blocks, int nblocks,
   std::vector<Tile> tiles[NBOX];
   long long off = 0, ioff = 0, doff = 0;
   std::vector<int> blk_cfg;
-  bool per_snap = false;
+  bool per_snap = false, faces = false;
   const double diss_scaling = std::pow(2.0, -2 * NG) * (NG % 2 == 0 ? -1 : 1);
   for (int b = 0; b < nblocks; ++b) {
     const z4c_block& in = blocks[b];
@@ -4184,6 +4285,7 @@ int z4c_set_blocks(z4c_ctx* c, const z4c_block* blocks, int nblocks,
     if ((long long)B.nis * NDV * 8 >= (long long)DV_DROP)
       return fail(Z4C_EINVAL, "set_blocks: block too large");
     B.faces = in.sommerfeld_faces & 63;
+    faces = faces || B.faces;
     B.pfaces = (in.sommerfeld_faces | in.outflow_faces) & 63;
     // stencil configuration until tuned: 256 threads (the fastest on 17^2,
     // 25^2 and 33^2 planes when measured), or 192 when the whole plane fits
@@ -4275,6 +4377,7 @@ int z4c_set_blocks(z4c_ctx* c, const z4c_block* blocks, int nblocks,
   HIPCALL(hipMemset(c->d1, 0, sizeof(double) * off * ND1));
   c->total_dv = doff;
   c->per_snap = per_snap;
+  c->faces = faces;
   c->blk_cfg = blk_cfg;
   c->hdev = hb;
   {
@@ -5197,7 +5300,7 @@ int z4c_rhs_form(z4c_ctx* c, int* rhs, int* step) {
   if (rc) return rc;
   if (!rhs || !step) return fail(Z4C_EINVAL, "rhs_form: null argument");
   *rhs = rhs_two(c) ? Z4C_FORM_TWO_PASSES : Z4C_FORM_ONE_KERNEL;
-  *step = Z4C_FORM_ONE_KERNEL;
+  *step = step_two(c) ? Z4C_FORM_TWO_PASSES : Z4C_FORM_ONE_KERNEL;
   return Z4C_OK;
 }
 
@@ -5252,6 +5355,15 @@ int ghost_update(z4c_ctx* c, double* u, int ghosts, hipStream_t s) {
   return rc;
 }
 
+// Whether the ghost update writes every ghost vertex from interior ones, so
+// that no ghost of the state before it is read: across levels (zero, then the
+// contributions), the exchange if every ghost has an owner, the periodic fill
+// of blocks that hold their images.
+bool update_fills_ghosts(const z4c_ctx* c, int ghosts) {
+  if (ghosts & 2) return c->ml || c->ext_nz == c->total_pts - c->total_int;
+  return (ghosts & 1) && !c->per_snap;
+}
+
 // ghosts: 0 holds the ghosts at u_n (AlgConstr(u_n), formed once); else the
 // ghost update of z4c_rk4_stage after every stage (1 single-block periodic
 // fill or 2 the exchange, plus 4 the physical fill), on the stage state whose
@@ -5266,28 +5378,42 @@ int launch_rk4_step(z4c_ctx* c, const z4c_params* p, double dt, double* u, doubl
   // bt_rk4 (task_list_integrators_butcher.cpp:37-49): subdiagonal of A and b
   static const double Asub[4] = {0.5, 0.5, 1.0, 0.0};
   static const double Bw[4] = {1. / 6., 1. / 3., 1. / 3., 1. / 6.};
-  // Every stage reads its neighbours' vertices, so no stage overwrites its
-  // input.  With ghosts held at u_n the states alternate between W0 and u
-  // (u_n is kept interior-indexed in W1), and both hold the ghosts
+  // In one kernel every stage reads its neighbours' vertices, so no stage
+  // overwrites its input.  With ghosts held at u_n the states alternate between
+  // W0 and u (u_n is kept interior-indexed in W1), and both hold the ghosts
   // AlgConstr(u_n) once stage 1 has read u_n's.  With a ghost update the
   // first three states alternate between W0 and W1, and u keeps u_n and its
-  // ghosts until the last stage.
-  double* const ins[4] = {u, W0, ghosts ? W1 : u, W0};
-  double* const outs[4] = {W0, ghosts ? W1 : u, W0, u};
-  // the ghost update across levels writes every ghost (zero, then the
-  // contributions), the periodic fill too: u_n's ghosts need no keeping
-  const bool all_ghosts = ((ghosts & 2) && c->ml) || ((ghosts & 1) && !c->per_snap);
+  // ghosts until the last stage.  In two passes without Sommerfeld faces every
+  // stage state overwrites u's interior (u_n is kept in W1 as well), and a ghost
+  // update finds u_n's ghosts in W0.
+  const bool two = p->cowling || step_two(c);
+  const bool inplace = two && !c->faces;
+  const bool held = !ghosts || inplace;  // u_n kept in W1, not in u
+  double* const outs[4] = {inplace ? u : W0, held ? u : W1, inplace ? u : W0, u};
+  const bool all_ghosts = update_fills_ghosts(c, ghosts);
+  auto copy_ghosts = [&](double* from, double* to) {
+    GhostArgs gc{c->d_blocks, launch_of(c, BOX_GHOST), from, to,
+                 p->eps_floor, p->tf_force_regularization, p->force_regularization};
+    PassTimer t(c, Z4C_PASS_GHOSTS, s);
+    hipLaunchKernelGGL(k_ghost_copy, dim3(grid_for(gc.L.ntiles)), dim3(TILE), 0, s, gc);
+    HIPCALL(hipGetLastError());
+    return (int)Z4C_OK;
+  };
+  if (ghosts && inplace && !all_ghosts) {
+    rc = copy_ghosts(u, W0);
+    if (rc) return rc;
+  }
   for (int st = 1; st <= 4; ++st) {
     FusedArgs a{};
-    a.u = ins[st - 1];
+    a.u = st == 1 ? u : outs[st - 2];
     a.mat = mat;
     a.o = rhs_params(p);
     a.sommerfeld = 1;
-    a.un = (!ghosts && st > 1) ? W1 : u;
-    a.un_int = !ghosts && st > 1;
+    a.un = (held && st > 1) ? W1 : u;
+    a.un_int = held && st > 1;
     a.acc = ACC;
     a.out = outs[st - 1];
-    a.keep = (!ghosts && st == 1) ? W1 : nullptr;
+    a.keep = (held && st == 1) ? W1 : nullptr;
     a.wa = Asub[st - 1] * dt;
     a.wb = Bw[st - 1] * dt;
     a.stage = st;
@@ -5296,18 +5422,15 @@ int launch_rk4_step(z4c_ctx* c, const z4c_params* p, double dt, double* u, doubl
     a.eps_floor = p->eps_floor;
     a.tf_force = p->tf_force_regularization;
     a.force_reg = p->force_regularization;
-    rc = launch_fused(c, a, s);
+    rc = launch_stage(c, p, two, a, s);
     if (rc) return rc;
     if (ghosts) {
       // SumBT's ghost values (u_n) into the stage state, then the ghost
       // update and AlgConstr of the whole block (z4c_rk4_stage's order)
       double* cur = a.out;
-      if (!all_ghosts && cur != u) {
-        GhostArgs gc{c->d_blocks, launch_of(c, BOX_GHOST), u, cur,
-                     p->eps_floor, p->tf_force_regularization, p->force_regularization};
-        PassTimer t(c, Z4C_PASS_GHOSTS, s);
-        hipLaunchKernelGGL(k_ghost_copy, dim3(grid_for(gc.L.ntiles)), dim3(TILE), 0, s, gc);
-        HIPCALL(hipGetLastError());
+      if (!all_ghosts && (inplace ? st > 1 : cur != u)) {
+        rc = copy_ghosts(inplace ? W0 : u, cur);
+        if (rc) return rc;
       }
       rc = ghost_update(c, cur, ghosts, s);
       if (!rc) rc = launch_alg(c, p, cur, nullptr, 0, s);
@@ -5316,7 +5439,10 @@ int launch_rk4_step(z4c_ctx* c, const z4c_params* p, double dt, double* u, doubl
       GhostArgs ga{c->d_blocks, launch_of(c, BOX_GHOST), u, W0, p->eps_floor,
                    p->tf_force_regularization, p->force_regularization};
       PassTimer t(c, Z4C_PASS_GHOSTS, s);
-      hipLaunchKernelGGL(k_rk4_ghosts, dim3(grid_for(ga.L.ntiles)), dim3(TILE), 0, s, ga);
+      if (inplace)
+        hipLaunchKernelGGL(k_rk4_ghosts_inplace, dim3(grid_for(ga.L.ntiles)), dim3(TILE), 0, s, ga);
+      else
+        hipLaunchKernelGGL(k_rk4_ghosts, dim3(grid_for(ga.L.ntiles)), dim3(TILE), 0, s, ga);
       HIPCALL(hipGetLastError());
     }
   }
@@ -5380,7 +5506,7 @@ int launch_ls_step(z4c_ctx* c, const z4c_params* p, const z4c_ls_tableau* T, dou
     a.ls_w[2] = T->gamma_2[st - 1];
     a.ls_w[3] = T->beta[st - 1] * dt;  // dt_scaled (time_integrators.hpp:37-40)
     a.ls_last = st == T->nstages;
-    rc = launch_fused(c, a, s);
+    rc = launch_stage(c, p, p->cowling || step_two(c), a, s);
     if (rc) return rc;
     if (ghosts) {
       rc = ghost_update(c, nxt, ghosts, s);

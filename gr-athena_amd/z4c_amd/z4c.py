@@ -429,7 +429,7 @@ class Z4c:
     RHS_FORMS = {"auto": 0, "one kernel": 1, "two passes": 2}
 
     def set_rhs_form(self, form):
-        """Form of Z4cRHS and the stage calls: "auto" (the faster one for
+        """Form of the right-hand sides and stages: "auto" (the faster one for
         the blocks), "one kernel" or "two passes"; results are the same."""
         check(self.L.z4c_set_rhs_form(self._ctx, self.RHS_FORMS[form]), "set_rhs_form")
 

@@ -463,12 +463,12 @@ int z4c_weyl(z4c_ctx* ctx, const z4c_params* p, const double* u, const double* a
    per brick of vertices, or a stencil pass into derivative slots and an algebra
    pass.  Results are equal bit for bit.  Z4C_FORM_AUTO (the default, restored by
    z4c_set_blocks) takes the faster one for the registered blocks; the others
-   hold for every later z4c_rhs and stage call of the context.  Whatever the
+   hold for every later z4c_rhs, stage call and step of the context.  Whatever the
    form, a right-hand side written over its own input takes two passes and a
    zero one (cowling) neither. */
 enum { Z4C_FORM_AUTO = 0, Z4C_FORM_ONE_KERNEL = 1, Z4C_FORM_TWO_PASSES = 2 };
 int z4c_set_rhs_form(z4c_ctx* ctx, int form);
-/* The forms that z4c_rhs and the stage calls, and the fused steps, now
+/* The forms that z4c_rhs and the stage calls, and the fused steps (of more than one stage), now
    take. */
 int z4c_rhs_form(z4c_ctx* ctx, int* rhs, int* step);
 

@@ -140,3 +140,58 @@ def test_step_equals_stages(faces, ghosts):
         # outermost ghosts of a filled face amplify them (weights summing to 31)
         assert bool((d <= (1e-9 if ghosts else 1e-14) * s + 1e-300).all()), (q, (d / s).max())
     z.close()
+
+
+@pytest.mark.parametrize("n, nblocks, form", [
+    ((2, 2, 2), 1, "two passes"), ((4, 4, 4), 16, "two passes"), ((4, 64, 4), 64, "two passes"),
+    ((17, 5, 3), 500, "two passes"), ((16, 16, 16), 1, "one kernel"),
+    ((32, 32, 32), 1, "one kernel"), ((2, 2, 2), 1024, "one kernel"), ((8, 8, 64), 1, "one kernel")])
+def test_form_rule(n, nblocks, form):
+    """Batches at which one form is faster by a quarter and more take it, for
+    z4c_rhs and for the steps."""
+    z = Z4c([MeshBlockGeom(n, (0.1, 0.1, 0.1), (0.3, 0.2, 0.1))] * nblocks, Params())
+    assert z.rhs_form() == (form, form)
+    z.close()
+
+
+@pytest.mark.parametrize("faces", [0, 45])
+@pytest.mark.parametrize("ghosts", [dict(), dict(periodic=True), dict(physical=True)])
+@pytest.mark.parametrize("kw", [dict(), dict(cowling=1), dict(matter=True)])
+def test_steps_in_both_forms(faces, ghosts, kw):
+    """rk4_step_fused and ls_step in one kernel and in two passes (in place
+    without faces) on ragged blocks: the same bits, ghosts included."""
+    gs = _batch(faces)
+    matter = kw.get("matter")
+    z = Z4c(gs, Params(diss=0.02, damp_kappa1=0.02, cowling=kw.get("cowling", 0)))
+    host = [perturbed_flat(g, seed=30 + b) for b, g in enumerate(gs)]
+    mat = None
+    if matter:
+        gen = torch.Generator(device="cuda").manual_seed(6)
+        mat = 1e-2 * torch.randn(10 * z.total_points, dtype=torch.float64, device="cuda",
+                                 generator=gen)
+    calls = [lambda u: z.rk4_step_fused(0.004, u, z.make_step_work().fill_(7.0), mat, **ghosts)]
+    for name in ("rk1", "rk2", "rk3", "rk4"):
+        calls.append(lambda u, t=name: z.ls_step(t, 0.004, u, z.make_ls_work().fill_(7.0), mat,
+                                                 **ghosts))
+    for call in calls:
+        out = []
+        for form in ("one kernel", "two passes"):
+            z.set_rhs_form(form)
+            u = z.upload(host)
+            z.AlgConstr(u)
+            call(u)
+            out.append(u)
+        assert torch.equal(out[0], out[1])
+    z.close()
+
+
+def test_zero_right_hand_side_runs_no_stencils():
+    """cowling: a stage is a copy with weights; neither stencils nor bricks."""
+    z = Z4c([MeshBlockGeom.cube(32, 0.1, 0.3)], Params(cowling=1))
+    u = z.upload([perturbed_flat(z.blocks[0], seed=2)])
+    z.set_timing(True)
+    z.rk4_step_fused(0.01, u, z.make_step_work())
+    z.ls_step("rk3", 0.01, u, z.make_ls_work())
+    t = z.get_timing()
+    assert t["stencil"][1] == 0 and t["assembly"][1] == 7
+    z.close()
