@@ -687,6 +687,54 @@ __global__ void __launch_bounds__(TILE) k_rk4_ghosts_inplace(GhostArgs a) {
                   a.force_reg);
 }
 
+// Held ghosts of a low-storage stage: AlgConstr of a.u's into a.w0.  Fields that
+// AlgConstr leaves alone are the same in both states from the second stage on.
+template <bool ALL>
+__global__ void __launch_bounds__(TILE) k_ls_ghosts(GhostArgs a) {
+  int b, i, j, k;
+  if (!tile_point(a.L, b, i, j, k)) return;
+  const DevBlock B = a.blocks[b];
+  const int N = B.npts;
+  const long long e = B.off * NVAR + flat(B, i, j, k);
+  const double* u = a.u + e;
+  double* w = a.w0 + e;
+  const bool reg = ALL || a.force_reg;  // chi and alpha change with force_reg only
+  double s[NVAR];
+#pragma unroll
+  for (int n = 0; n < NVAR; ++n) {
+    const bool alg = (n >= V_GXX && n < V_GXX + 6) || (n >= V_AXX && n < V_AXX + 6);
+    s[n] = ALL || alg || n == V_CHI || n == V_ALPHA ? u[(long long)n * N] : 0.0;
+  }
+  algconstr_vals(s + V_GXX, s + V_AXX, s[V_CHI], s[V_ALPHA], a.eps_floor, a.tf_force,
+                 a.force_reg);
+#pragma unroll
+  for (int n = 0; n < NVAR; ++n) {
+    const bool alg = (n >= V_GXX && n < V_GXX + 6) || (n >= V_AXX && n < V_AXX + 6);
+    if (ALL || alg || (reg && (n == V_CHI || n == V_ALPHA))) w[(long long)n * N] = s[n];
+  }
+}
+
+// Interior vertices of all fields from one state into another.
+struct CopyArgs {
+  const DevBlock* blocks;
+  Launch L;
+  const double* from;
+  double* to;
+};
+
+__global__ void __launch_bounds__(TILE) k_copy_interior(CopyArgs a) {
+  int b, i, j, k;
+  if (!tile_point(a.L, b, i, j, k)) return;
+  const DevBlock B = a.blocks[b];
+  const int N = B.npts;
+  const long long e = B.off * NVAR + flat(B, i, j, k);
+  double v[NVAR];
+#pragma unroll
+  for (int n = 0; n < NVAR; ++n) v[n] = a.from[e + (long long)n * N];
+#pragma unroll
+  for (int n = 0; n < NVAR; ++n) a.to[e + (long long)n * N] = v[n];
+}
+
 __global__ void __launch_bounds__(TILE) k_rk4_ghosts(GhostArgs a) {
   int b, i, j, k;
   if (!tile_point(a.L, b, i, j, k)) return;
@@ -3328,12 +3376,12 @@ void launch_stencil_cfg(int cfg, const StencilArgs& sa, hipStream_t s) {
 
 // Whether z4c_rhs runs in two passes, and the stages of a step: a stage in one
 // kernel pays for the second buffer that its state goes to, about 5 % of a
-// right-hand side.
+// right-hand side, and `extra` us.
 bool rhs_two(const z4c_ctx* c) {
   return c->form ? c->form == Z4C_FORM_TWO_PASSES : c->t_one >= c->t_two;
 }
-bool step_two(const z4c_ctx* c) {
-  return c->form ? c->form == Z4C_FORM_TWO_PASSES : c->t_one >= 0.95 * c->t_two;
+bool step_two(const z4c_ctx* c, double extra = 0.0) {
+  return c->form ? c->form == Z4C_FORM_TWO_PASSES : c->t_one + extra >= 0.95 * c->t_two;
 }
 
 // The derivative slots, allocated by the first two-pass right-hand side.
@@ -5468,25 +5516,35 @@ int check_ls(const z4c_ls_tableau* t, bool need_2s, const char* what) {
   return Z4C_OK;
 }
 
-// Fused low-storage step: the stage states alternate between u and the second
-// work register (a stage reads its neighbours' vertices), each stage's output
-// first receiving its input's ghosts; u1 lives interior-indexed in work.
+// Fused low-storage step.  In one kernel a stage reads its neighbours'
+// vertices, so the stage states alternate between u and the second work
+// register W; an odd number of stages ends with the interior copied from W.  In
+// two passes without Sommerfeld faces every stage overwrites u's interior.  u1
+// lives interior-indexed in work.  A stage's output receives its input's ghosts
+// where the ghost update does not write them all; with held ghosts it receives
+// AlgConstr of them (the update leaves ghosts alone; AlgConstr of the whole block
+// reaches them after every stage), in one pass.
 int launch_ls_step(z4c_ctx* c, const z4c_params* p, const z4c_ls_tableau* T, double dt,
                    double* u, double* work, const double* mat, int ghosts, hipStream_t s) {
-  const long long n = c->total_pts * NVAR;
   double* U1 = work;
-  double* W = work + n;
+  double* W = work + c->total_pts * NVAR;
+  const bool all_ghosts = update_fills_ghosts(c, ghosts);
+  // In two passes without faces the interior copy (0.03 us per 256 vertices) and
+  // the ghost copies (0.026 us) fall away: a stage's share of them counts against
+  // the one kernel.
+  const int odd = T->nstages & 1;
+  double extra = 0.0;
+  if (!c->faces) {
+    extra = odd * 0.03 * c->ntiles[BOX_INTERIOR];
+    if (ghosts && !all_ghosts) extra += (T->nstages - odd) * 0.026 * c->ntiles[BOX_GHOST];
+    extra /= T->nstages;
+  }
+  const bool two = p->cowling || step_two(c, extra);
+  const bool inplace = two && !c->faces;
   double* cur = u;
   int rc = Z4C_OK;
   for (int st = 1; st <= T->nstages; ++st) {
-    double* nxt = cur == u ? W : u;
-    {
-      GhostArgs gc{c->d_blocks, launch_of(c, BOX_GHOST), cur, nxt, p->eps_floor,
-                   p->tf_force_regularization, p->force_regularization};
-      PassTimer t(c, Z4C_PASS_GHOSTS, s);
-      hipLaunchKernelGGL(k_ghost_copy, dim3(grid_for(gc.L.ntiles)), dim3(TILE), 0, s, gc);
-      HIPCALL(hipGetLastError());
-    }
+    double* nxt = inplace || cur == W ? u : W;
     FusedArgs a{};
     a.u = cur;
     a.mat = mat;
@@ -5506,27 +5564,38 @@ int launch_ls_step(z4c_ctx* c, const z4c_params* p, const z4c_ls_tableau* T, dou
     a.ls_w[2] = T->gamma_2[st - 1];
     a.ls_w[3] = T->beta[st - 1] * dt;  // dt_scaled (time_integrators.hpp:37-40)
     a.ls_last = st == T->nstages;
-    rc = launch_stage(c, p, p->cowling || step_two(c), a, s);
+    rc = launch_stage(c, p, two, a, s);
     if (rc) return rc;
-    if (ghosts) {
+    GhostArgs ga{c->d_blocks, launch_of(c, BOX_GHOST), cur, nxt, p->eps_floor,
+                 p->tf_force_regularization, p->force_regularization};
+    const dim3 gg(grid_for(ga.L.ntiles));
+    if (st == T->nstages && nxt == W) {
+      // u's ghosts are the ones this stage read
+      const CopyArgs ca{c->d_blocks, launch_of(c, BOX_INTERIOR), W, u};
+      hipLaunchKernelGGL(k_copy_interior, dim3(grid_for(ca.L.ntiles)), dim3(TILE), 0, s, ca);
+      HIPCALL(hipGetLastError());
+      nxt = u;
+    }
+    if (!ghosts) {
+      PassTimer t(c, Z4C_PASS_GHOSTS, s);
+      if (cur == nxt)
+        hipLaunchKernelGGL(k_rk4_ghosts_inplace, gg, dim3(TILE), 0, s, ga);
+      else if (st == 1)
+        hipLaunchKernelGGL(k_ls_ghosts<true>, gg, dim3(TILE), 0, s, ga);
+      else
+        hipLaunchKernelGGL(k_ls_ghosts<false>, gg, dim3(TILE), 0, s, ga);
+      HIPCALL(hipGetLastError());
+    } else {
+      if (cur != nxt && !all_ghosts) {
+        PassTimer t(c, Z4C_PASS_GHOSTS, s);
+        hipLaunchKernelGGL(k_ghost_copy, gg, dim3(TILE), 0, s, ga);
+        HIPCALL(hipGetLastError());
+      }
       rc = ghost_update(c, nxt, ghosts, s);
       if (!rc) rc = launch_alg(c, p, nxt, nullptr, 0, s);
       if (rc) return rc;
-    } else {
-      // the update leaves ghosts alone; AlgConstr of the whole block
-      // reaches them after every stage
-      GhostArgs ga{c->d_blocks, launch_of(c, BOX_GHOST), nxt, nullptr, p->eps_floor,
-                   p->tf_force_regularization, p->force_regularization};
-      PassTimer t(c, Z4C_PASS_GHOSTS, s);
-      hipLaunchKernelGGL(k_rk4_ghosts_inplace, dim3(grid_for(ga.L.ntiles)), dim3(TILE), 0, s,
-                         ga);
-      HIPCALL(hipGetLastError());
     }
     cur = nxt;
-  }
-  if (cur != u) {
-    hipLaunchKernelGGL(k_copy, dim3(elementwise_grid(n)), dim3(256), 0, s, u, (const double*)cur, n);
-    HIPCALL(hipGetLastError());
   }
   return Z4C_OK;
 }

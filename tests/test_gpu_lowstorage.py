@@ -132,6 +132,83 @@ def test_ls_step_periodic_gauge_wave():
     z.close()
 
 
+def _ghost_passes(z, name, u, **ghosts):
+    z.get_timing()
+    z.set_timing(True)
+    z.ls_step(name, 0.001, u, z.make_ls_work(), **ghosts)
+    z.set_timing(False)
+    return z.get_timing()["ghosts"][1]
+
+
+@pytest.mark.parametrize("form", ["one kernel", "two passes"])
+def test_ls_step_passes_over_the_ghosts(form):
+    """Passes over all ghosts, each about a quarter of a stage on 16^3 blocks:
+    one a stage where they are held, none where the ghost update writes them
+    all, and one for each state but the last that an open box's update leaves
+    some of."""
+    p = Params(**MP_GAUGE)
+    n = 6
+    gs = [MeshBlockGeom.cube(n, 1.0, tuple(float(n * (b >> d & 1)) for d in range(3)))
+          for b in range(8)]
+    z = Z4c(gs, p)
+    z.set_rhs_form(form)
+    u = z.upload(_states(gs, p))
+    for name, nst in (("rk1", 1), ("rk3", 3), ("rk4", 4)):
+        assert _ghost_passes(z, name, u) == nst
+        assert _ghost_passes(z, name, u, periodic=True) == 0
+    z.set_exchange(0.0, 2.0 * n, True)
+    for name in ("rk1", "rk3", "rk4"):
+        assert _ghost_passes(z, name, u, exchange=True) == 0
+    z.set_exchange(0.0, 2.0 * n, False)
+    for name, copies in (("rk1", 0), ("rk3", 2), ("rk4", 4)):
+        assert _ghost_passes(z, name, u, exchange=True) == (copies if form == "one kernel" else 0)
+    z.close()
+
+
+@pytest.mark.parametrize("periodic", [True, False, (True, False, True)])
+@pytest.mark.parametrize("form", ["one kernel", "two passes"])
+def test_ls_step_with_exchange_equals_stages(form, periodic):
+    """The exchange after every stage where it writes every ghost (a periodic
+    box) and where it leaves some: the stage sequence's bits.  The work
+    registers start as NaN: no ghost of theirs may be read unwritten."""
+    p = Params(**MP_GAUGE)
+    n = 6
+    gs = [MeshBlockGeom.cube(n, 0.1, tuple(0.1 * n * (b >> d & 1) for d in range(3)))
+          for b in range(8)]
+    z = Z4c(gs, p)
+    z.set_exchange(0.0, 0.2 * n, periodic)
+    us = _states(gs, p, seed=8)
+    for name in NAMES:
+        ua, ub = z.upload(us), z.upload(us)
+        z.set_rhs_form("auto")
+        z.ls_step_stages(name, 0.002, ua, z.zeros(), z.zeros(), exchange=True)
+        z.set_rhs_form(form)
+        z.ls_step(name, 0.002, ub, z.make_ls_work().fill_(float("nan")), exchange=True)
+        assert torch.equal(ua, ub), name
+    z.close()
+
+
+@pytest.mark.parametrize("force", [0, 1])
+def test_ls_step_held_ghosts_with_floors(force):
+    """Held ghosts receive AlgConstr once a stage, chi and the lapse floored
+    with force_regularization: the stage sequence's bits."""
+    g = MeshBlockGeom.cube((9, 6, 7), 0.1, 0.3)
+    p = Params(force_regularization=force, eps_floor=0.05, **MP_GAUGE)
+    (u,) = _states([g], Params(**MP_GAUGE), seed=3)
+    u[0] = np.where(np.arange(u[0].size).reshape(u[0].shape) % 3 == 0, 0.01, u[0])
+    z = Z4c([g], p)
+    for name in NAMES:
+        ua, ub = z.upload([u]), z.upload([u])
+        z.ls_step_stages(name, 0.002, ua, z.zeros(), z.zeros())
+        z.set_rhs_form("one kernel")
+        z.ls_step(name, 0.002, ub, z.make_ls_work().fill_(float("nan")))
+        z.set_rhs_form("auto")
+        torch.cuda.synchronize()
+        assert torch.equal(torch.isnan(ua), torch.isnan(ub))
+        assert torch.equal(torch.nan_to_num(ua), torch.nan_to_num(ub)), name
+    z.close()
+
+
 def test_ls_rejects_bad_input():
     from z4c_amd._capi import LsTableau, Z4cError
     g = MeshBlockGeom.cube(8, 0.1, 0.0)
