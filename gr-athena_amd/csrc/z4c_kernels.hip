@@ -1048,9 +1048,10 @@ struct ConArgs {
   double chi_psi_power, chi_div_floor, r_max_con;
 };
 
-// Two waves a SIMD although 67 registers spill (328 unbounded, one wave): the
-// loads' latency costs more, 2.03 -> 1.92 ms for 400 uneven blocks.
-__global__ void __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(2)))
+// WAVES 2: two waves a SIMD although 67 registers spill (324 unbounded, one
+// wave); z4c_adm_constraints says when.
+template <int WAVES>
+__global__ void __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(WAVES)))
 k_constraints(ConArgs a) {
   int b, i, j, k;
   if (!tile_point(a.L, b, i, j, k)) return;
@@ -4538,7 +4539,15 @@ int z4c_adm_constraints(z4c_ctx* c, const z4c_params* p, const double* u,
   if (rc) return rc;
   ConArgs a{c->d_blocks, launch_of(c, BOX_INTERIOR), u, adm, mat, c->d1, con,
             p->chi_psi_power, p->chi_div_floor, p->r_max_con};
-  hipLaunchKernelGGL(k_constraints, dim3(grid_for(a.L.ntiles)), dim3(TILE), 0, s, a);
+  // Two waves a SIMD hide the loads' latency of a full chip (2.03 -> 1.92 ms for
+  // 400 uneven blocks, whole call 1531 -> 1458 us for 320 of 16^3) and of workgroups
+  // just over one a CU (16 of 16^3: 79 -> 75 us); a single round pays the spills
+  // for nothing (one 8^3 or 32^3 block: 34.7 -> 38.2, 41.4 -> 47.4 us), and between
+  // two and six rounds neither is better throughout (64 of 16^3: 297 -> 304 us, a
+  // 64^3 block: 173 -> 167).
+  const int n = a.L.ntiles, cu = c->n_cu;
+  const bool two = n >= 6 * cu || (n > cu && n <= cu + cu / 3);
+  hipLaunchKernelGGL(two ? k_constraints<2> : k_constraints<1>, dim3(grid_for(n)), dim3(TILE), 0, s, a);
   HIPCALL(hipGetLastError());
   return Z4C_OK;
 }

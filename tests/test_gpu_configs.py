@@ -458,3 +458,22 @@ def test_multilevel_octree_step_graph_equals_stage_sequence():
     assert torch.equal(ug, ug2)
     assert torch.equal(ug, us), float((ug - us).abs().max())
     z.close()
+
+
+def test_constraints_of_a_block_do_not_depend_on_the_batch():
+    """The constraint kernel of small and of large batches (two register
+    budgets): the same bits for the same block."""
+    g = [MeshBlockGeom.cube(8, 0.1, 0.3)]
+    out = []
+    for n in (1, 90, 160, 520):  # 3, 270, 480 and 1560 workgroups
+        z = Z4c(g * n, Params(chi_div_floor=1e-5))
+        host = perturbed_flat(g[0], seed=4, amp=(1e-3, 1e-1))
+        u = torch.from_numpy(host).to("cuda").reshape(1, -1).repeat(n, 1).reshape(-1)
+        z.AlgConstr(u)
+        adm, con = z.zeros(17), z.zeros(7)
+        z.Z4cToADM(u, adm)
+        z.ADMConstraints(con, adm, None, u)
+        out.append(con.view(n, -1).clone())
+        z.close()
+    for c in out:
+        assert bool((c == out[0]).all())
