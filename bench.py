@@ -32,13 +32,11 @@ import numpy as np  # noqa: E402
 PEAK_FP64 = 78.6e12   # FP64 vector, FMA counted as two operations
 PEAK_FP64_NOFMA = 39.3e12  # the same issue rate when every operation is a separate add or mul
 PEAK_HBM = 8.0e12
-# kernel of each timed pass (the stencil and assembly passes are the two parts,
-# 57:43, of the time of one kernel), and the committed counter summary holding the
+# kernel of each timed pass, and the committed counter summary holding the
 # measured HBM bytes per launch of each kernel (FETCH_SIZE / WRITE_SIZE
 # passes, calibrated against a copy kernel of known size)
-PASS_KERNEL = {"stencil": "k_fused", "assembly": "k_fused",
+PASS_KERNEL = {"stage": "k_fused", "stencil": "k_stencil", "assembly": "k_rk4_stage",
                "ghosts": "k_rk4_ghosts", "prepare": "k_prep"}
-PASS_SHARE = {"stencil": 0.57, "assembly": 0.43}
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "z4c_rk4_step_2048blocks_pmc.md")
 
 # FLOPs of one block of n^3 cells, counted exactly by the FLOP-counting build
@@ -69,14 +67,17 @@ B_RHS = 2 * 22 * 8
 
 
 def pass_flops(name, blocks):
-    """Algorithmic FLOPs of one launch of a pass over ``blocks``: the
-    stencil part carries the stencil share of one RHS; the assembly part
-    (curvature, assembly, stage update, AlgConstr) a quarter of the rest of
-    the step; the other passes carry data movement only."""
+    """Algorithmic FLOPs of one launch of a pass over ``blocks``: a stage in
+    one kernel carries a quarter of the step; in two passes the stencil pass
+    carries the stencil share of one RHS and the assembly (curvature,
+    assembly, stage update, AlgConstr) a quarter of the rest of the step; the
+    other passes carry data movement only."""
     tot = 0
     for g in blocks:
         st, _, step = FLOPS_BLOCK[g.nx[0]]
-        if name == "stencil":
+        if name == "stage":
+            tot += step / 4.0
+        elif name == "stencil":
             tot += st
         elif name == "assembly":
             tot += (step - 4 * st) / 4.0
@@ -119,7 +120,7 @@ def parse():
     ap.add_argument("--no-perblock", action="store_true", help="skip the per-block launch comparison")
     ap.add_argument("--cpu-seconds", type=float, default=15.0)
     ap.add_argument("--no-tune", action="store_true",
-                    help="keep the default stencil plan (no autotuner trial launches, e.g. under a profiler)")
+                    help="no effect: the step's stages run in one kernel, which has no tuned plan")
     ap.add_argument("--no-adjoint", action="store_true", help="skip the adjoint cost leg")
     ap.add_argument("--no-sensitivity", action="store_true",
                     help="skip the 100-step evolution + 10-step adjoint sensitivity leg")
@@ -249,11 +250,8 @@ def main():
     dt = min(z.NewBlockTimeStep(0.25), 1.0)
     torch.cuda.synchronize()
     log("initial data ready")
-    t_tune = time.perf_counter()
-    plan = z.stencil_plan() if args.no_tune else z.autotune(u, reps=3)
-    log(f"stencil workgroup sizes by block size ("
-        + ("default plan" if args.no_tune else f"autotuned in {time.perf_counter() - t_tune:.2f} s")
-        + "): " + ", ".join(f"{'x'.join(map(str, k))}: {v}" for k, v in sorted(plan.items())))
+    form = z.rhs_form()[1]
+    log(f"stages in {form}")
 
     def step():
         # the fused step replayed from its HIP graph (captured on first use)
@@ -281,6 +279,10 @@ def main():
     T_eager = time.perf_counter() - t1
     z.set_timing(False)
     passes = z.get_timing()
+    if form == "one kernel":
+        # the timer divides the time of each launch between two passes
+        st, asm = passes.pop("stencil"), passes.pop("assembly")
+        passes = {"stage": (st[0] + asm[0], st[1]), **passes}
     log(f"{args.steps} eager steps with pass timers in {T_eager:.3f} s")
     pinfo = {}
     step_f = step_flops(blocks)
@@ -290,10 +292,11 @@ def main():
         avg = ms / n * 1e-3
         e = {"launches": n, "avg_ms": avg * 1e3}
         fl = pass_flops(name, blocks)
-        # algorithmic bytes of the pass: the stencil part reads the 22
-        # fields once per owned point; the assembly part moves the rest of a
-        # stage's share of the 2992 B per owned point-step
-        bts = {"stencil": 22 * 8.0 * owned, "assembly": (B_STEP / 4.0 - 22 * 8.0) * owned}.get(name)
+        # algorithmic bytes of the pass: a stage's share of the 2992 B per
+        # owned point-step; in two passes the stencil pass reads the 22 fields
+        # once per owned point and the assembly moves the rest
+        bts = {"stage": B_STEP / 4.0 * owned, "stencil": 22 * 8.0 * owned,
+               "assembly": (B_STEP / 4.0 - 22 * 8.0) * owned}.get(name)
         if fl > 0:
             e["alg_flops"] = fl
             e["tflops"] = fl / avg / 1e12
@@ -304,7 +307,6 @@ def main():
             e["frac_hbm"] = bts / avg / PEAK_HBM
         tr = measured_traffic(PASS_KERNEL.get(name, ""))
         if tr:
-            tr *= PASS_SHARE.get(name, 1.0)
             e["measured_traffic_bytes"] = tr
             e["measured_gbs"] = tr / avg / 1e9
         pinfo[name] = e
@@ -324,8 +326,7 @@ def main():
                                "per stage",
                    "nblocks": len(blocks), "owned_points": owned,
                    "interior_points": interior_pts, "padded_points": z.total_points,
-                   "parallelism": "single GPU",
-                   "stencil_threads": {"x".join(map(str, k)): v for k, v in sorted(plan.items())}},
+                   "parallelism": "single GPU", "stage_form": form},
     }
     # roofline of the dominant kernel (largest total time): algorithmic FLOPs
     # (counted, FLOPS_BLOCK) and bytes per launch over its event-timed
@@ -497,7 +498,6 @@ def multilevel_run(adm_fn, params, nsteps=100, nblocks=2048):
     z.AlgConstr(u)
     dt = min(g.dx[0] for g in blocks) * 0.25
     work = z.make_step_work()
-    z.autotune(u, reps=2)
     z.rk4_step_fused(dt, u, work, graph=True, exchange=True, physical=True)
     torch.cuda.synchronize()
     t0 = time.perf_counter()
@@ -575,7 +575,6 @@ def sensitivity_run(adm_fn, params, nsteps=100, window=10, tree="independent", f
         z.physical_bc(u0)
         z.AlgConstr(u0)
     dt = min(z.NewBlockTimeStep(0.25), 1.0)
-    z.autotune(u0, reps=2)
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     res = hamiltonian_sensitivity(z, u0, dt, nsteps, window, exchange=ghosts, physical=ghosts)
@@ -749,7 +748,7 @@ def per_block(z, blocks, params, u, dt, owned):
     return {"value": owned * n / T, "unit": "point-updates/s", "steps": n,
             "ms_per_step": T / n * 1e3,
             "form": "per-block launches: 2048 single-block contexts, one fused rk4 step "
-                    "(14 kernel launches) per block per step"}
+                    "(5 kernel launches: four stages, the ghosts) per block per step"}
 
 
 if __name__ == "__main__":
