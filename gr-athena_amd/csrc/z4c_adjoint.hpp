@@ -23,11 +23,16 @@
 #include "z4c_device.hpp"
 #include "z4c_rhs_point.hpp"
 
-// Fused multiply-adds in the adjoint only: the reference has no derivative code
-// whose rounding these kernels would have to follow (the right-hand side and
-// the stencils it is linearised with keep the reference's separate roundings).
-// 64 cotangents of a 32^3 block 8.83 -> 8.44 ms, a step of 320 blocks of 16^3
-// 47.1 -> 44.5 ms; error against 64-bit autograd as before.
+// Fused multiply-adds in this header: the reference has no derivative code whose
+// rounding the adjoint would have to follow.  The right-hand side and the stencils
+// that it is linearised with keep the reference's separate roundings; the forward
+// intermediates formed here do not, so Ht of z4c_hamiltonian_norm, which is formed
+// from them, differs from the right-hand side's by rounding (where its terms cancel
+// completely, by all that is left).  64 cotangents of a 32^3 block 8.83 -> 8.44 ms,
+// a step of 320 blocks of 16^3 47.1 -> 44.5 ms; error against 64-bit autograd as
+// before.  With separate roundings in the forward part alone k_adj_fwd spills 68
+// registers or drops to one wave: the norm takes 12 % longer (320 blocks of 16^3
+// 1.58 -> 1.76 ms), the same step's adjoint 2 %.
 #pragma clang fp contract(fast)
 namespace z4c {
 

@@ -9,7 +9,8 @@
 // the threads write to LDS in between (the mixed derivatives are the
 // reference's nested Dx(a, Dx(b, u)), a < b).  The algebra takes each field's
 // derivatives as they come, so that at most about 100 values of the vertex are
-// live: 256 VGPRs, no spills, two waves per SIMD.
+// live: 256 VGPRs without a vector spill, two waves per SIMD (87 scalars wait in
+// lanes of vector registers).
 //
 // Against the two-pass form (stencil pass writing 106 values a vertex, algebra
 // pass reading them back: 67 GB of HBM traffic per stage of 2048 blocks of
@@ -77,12 +78,12 @@ struct FusedArgs {
   const DevBlock* blocks;
   const FusedTile* tiles;
   int ntiles;
-  const double* u;    // state read (never written by the kernel's own launch
-                      // except at the vertices' own place, `out` == u is not allowed)
+  const double* u;    // state read; rhs and out lie apart from it (every brick reads its
+                      // neighbours' vertices).  In two passes out may be u itself
   const double* mat;  // may be null
   RhsParams o;
-  int cowling;        // zero right-hand side
-  int sommerfeld;     // apply the Sommerfeld rows on flagged faces
+  int cowling;        // zero right-hand side (two passes only)
+  int sommerfeld;     // apply the Sommerfeld rows on flagged faces (two passes: always)
   double* rhs;        // right-hand side (null: stage update)
   // stage update
   const double* un;

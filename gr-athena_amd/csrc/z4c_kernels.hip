@@ -658,7 +658,9 @@ k_rk4_stage(StageArgs a) {
 // applies AlgConstr to the state's ghosts once (after the first stage has
 // read them), and copies them into the work register that the stages alternate
 // with.  The 30.3 M ghost vertices of 2048 blocks of 16^3 .. 32^3 cells: 18.8 GB
-// (8.9 read, 9.9 written; ghost rows of 32 bytes) in 2.9 to 5.4 ms a step.
+// (8.9 read, 9.9 written; ghost rows of 32 bytes) in 5.4 ms a step, against 2.0 ms
+// for AlgConstr in place (k_rk4_ghosts_inplace: steps in two passes), which is what
+// the one kernel pays for its second buffer.
 struct GhostArgs {
   const DevBlock* blocks;
   Launch L;

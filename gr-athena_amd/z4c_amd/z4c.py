@@ -313,8 +313,8 @@ class Z4c:
 
     def rk4_step_fused(self, dt, u, work, mat=None, stream=None, graph=False, periodic=False,
                        exchange=False, physical=False):
-        """One bt_rk4 step, fused per stage (RHS assembly + SumBT + AlgConstr
-        in one kernel).  Without a ghost update the ghosts are held at u_n
+        """One bt_rk4 step, fused per stage (SumBT and AlgConstr where the RHS is
+        assembled).  Without a ghost update the ghosts are held at u_n
         and the state equals ``rk4_step`` with no ghost update; with
         ``periodic`` / ``exchange`` / ``physical`` every stage updates the
         ghosts as ``rk4_step`` with the same flags does, then applies

@@ -313,18 +313,16 @@ int z4c_rk4_stage(z4c_ctx* ctx, const z4c_params* p, int stage, double dt,
    (src/task_list/gr/task_list_gr_z4c.cpp:45-89 over stages 1..4, tableau
    src/task_list/task_list_integrators_butcher.cpp:37-49) on all blocks, with
    ghost vertices held at u_n (no exchange) and Sommerfeld faces honoured.
-   Per stage: the stencil pass of Z4cRHS, then one kernel that forms the
-   curvature part, assembles the RHS and applies SumBT and AlgConstr at each
-   interior vertex; the ghosts get AlgConstr(u_n) once.  The derivative
+   Per stage: the right-hand side, SumBT and AlgConstr at each interior
+   vertex, in one kernel or in a stencil pass and an algebra pass
+   (z4c_set_rhs_form); the ghosts get AlgConstr(u_n) once.  The derivative
    arrays of PrepareZ4cDerivatives are not formed (nothing in the step reads
    them; z4c_adm_constraints prepares its own).  The state equals
    z4c_rk4_stage over stages 1..4 (same sums in the same order) without k
    registers: `work` is caller-owned device memory of 3 * 22 * elems_per_var
-   doubles.  Without Sommerfeld faces every stage state is written over the
-   interior of `u`, as the reference's stage update overwrites its state
-   (work then holds u_n and the running sum); with them the stage states
-   alternate between two work registers.  `u` holds u_n on entry and
-   u_{n+1} on return. */
+   doubles, all of it scratch (stage states, u_n, the running sum): which of
+   `u` and work a stage state is written to depends on the form and on
+   Sommerfeld faces.  `u` holds u_n on entry and u_{n+1} on return. */
 int z4c_rk4_step(z4c_ctx* ctx, const z4c_params* p, double dt, double* u,
                  double* work, const double* mat, void* stream);
 
@@ -385,17 +383,16 @@ int z4c_ls_stage(z4c_ctx* ctx, const z4c_params* p, const z4c_ls_tableau* t, int
                  double dt, double* u, double* u1, const double* u2, double* rhs,
                  const double* mat, int ghosts, void* stream);
 
-/* One whole low-storage step, fused per stage like z4c_rk4_step: the
-   stencil pass, then one kernel forming the right-hand side, the two
-   weighted averages, AddZ4cRHS and AlgConstr at each interior vertex (the
-   sums and their order of z4c_ls_stage).  `ghosts` = 0 holds the ghosts
+/* One whole low-storage step, fused per stage like z4c_rk4_step: right-hand
+   side, the two weighted averages, AddZ4cRHS and AlgConstr at each interior
+   vertex (the sums and their order of z4c_ls_stage).  `ghosts` = 0 holds the ghosts
    out of the update (WeightedAve and AddZ4cRHS act on interior vertices),
    with AlgConstr applied to them after every stage; otherwise the ghost
    update of z4c_ls_stage (1 periodic fill or 2 exchange, plus 4 physical
    fill) and AlgConstr of the whole block after every stage.  The
    derivative arrays are not prepared.  `work` is caller-owned device
-   memory of 2 * 22 * elems_per_var doubles (u1, and a second state buffer
-   that Sommerfeld faces need).  2S tableaus only (every gamma_3 == 0, as
+   memory of 2 * 22 * elems_per_var doubles (u1, and a second state buffer),
+   both always needed.  2S tableaus only (every gamma_3 == 0, as
    for every integrator GR_Z4c accepts).  `u` holds u_n on entry and
    u_{n+1} on return. */
 int z4c_ls_step(z4c_ctx* ctx, const z4c_params* p, const z4c_ls_tableau* t, double dt,
@@ -554,7 +551,9 @@ int z4c_rk4_step_ghosts_vjp(z4c_ctx* ctx, const z4c_params* p, double dt, const 
    src/outputs/history.cpp:178-205) of dx*dy*dz*Ht^2.  The objective of the
    adjoint sensitivity runs (the reference's H-norm2 column integrates the
    H of ADMConstraints, the same constraint discretised through the ADM
-   variables).  Waits for the stream; J is host memory. */
+   variables).  Ht is formed with fused multiply-adds, so it equals the
+   right-hand side's to rounding, not bit for bit.  Waits for the stream; J is
+   host memory. */
 int z4c_hamiltonian_norm(z4c_ctx* ctx, const z4c_params* p, const double* u, double* J,
                          void* stream);
 /* ubar (one register of 22 * elems_per_var doubles) = dJ/du at every vertex. */

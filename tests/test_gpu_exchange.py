@@ -190,7 +190,7 @@ def test_sommerfeld_block_evolution_with_physical_fill():
 
 def _fused_vs_stages(gs, params, host, dt, nsteps, setup=None, **flags):
     """The fused step with a ghost update against rk4_step (four
-    z4c_rk4_stage calls) with the same update."""
+    z4c_rk4_stage calls, right-hand sides in two passes) with the same update."""
     z = Z4c(gs, params)
     if setup:
         setup(z)
@@ -199,7 +199,9 @@ def _fused_vs_stages(gs, params, host, dt, nsteps, setup=None, **flags):
     work = z.make_step_work()
     z.PrepareZ4cDerivatives(ua)
     for _ in range(nsteps):
+        z.set_rhs_form("two passes")
         z.rk4_step(dt, ua, un, k, **flags)
+        z.set_rhs_form("one kernel")
         z.rk4_step_fused(dt, ub, work, **flags)
     torch.cuda.synchronize()
     A, Bf = z.download(ua, 22), z.download(ub, 22)
@@ -212,8 +214,7 @@ def _fused_vs_stages(gs, params, host, dt, nsteps, setup=None, **flags):
 
 def test_fused_step_with_exchange_equals_stage_sequence():
     """Split periodic gauge wave (2 x 1 x 2 blocks): the fused step with the
-    exchange after every stage (stages in place) against the stage
-    sequence, two steps."""
+    exchange after every stage against the stage sequence, two steps."""
     n = 16
     gs = _grid((2, 1, 2), n, 1.0 / n, -0.5)
     params = Params(lapse_oplog=2.0, shift_Gamma=1.0, shift_eta=2.0, diss=0.02,
@@ -239,8 +240,8 @@ def test_fused_step_with_periodic_fill_equals_stage_sequence():
 
 @pytest.mark.parametrize("faces,outflow", [(63, 0), (0, 63)])
 def test_fused_step_with_physical_fill_equals_stage_sequence(faces, outflow):
-    """Physical ghost fill after every stage: with Sommerfeld faces (stage
-    states in the work registers) and with outflow faces only (in place)."""
+    """Physical ghost fill after every stage: with Sommerfeld faces and with
+    outflow faces only."""
     g = MeshBlockGeom.cube(12, 1.0 / 12, (0.3, -0.45, 0.2), faces=faces, outflow=outflow)
     p = Params(lapse_oplog=2.0, shift_Gamma=1.0, shift_eta=2.0, diss=0.02, damp_kappa1=0.02,
                chi_div_floor=1e-5)

@@ -2,8 +2,9 @@
 70% 16^3, 20% 24^3, 10% 32^3 cells, levels 0-7, Brill-Lindquist binary),
 through properties that do not depend on the size:
 
-* the fused in-place bt_rk4 step equals the four-stage sequence of the
-  GR_Z4c task list (z4c_rk4_stage) on every block to rounding;
+* the fused bt_rk4 step (one kernel a stage) equals the four-stage sequence of
+  the GR_Z4c task list (z4c_rk4_stage, right-hand sides in two passes) on every
+  block to rounding;
 * the right-hand side of the whole batch, at one block of each size class,
   equals the oracle's to the RHS tolerance (1e-12 of each variable's range);
 * restriction followed by whole-interior prolongation (the AMR refinement
@@ -51,7 +52,9 @@ def test_fused_step_equals_stage_sequence_full_size(workload):
     ub = u0.clone()
     un, k = z.make_rk_registers()
     z.PrepareZ4cDerivatives(ua)
+    z.set_rhs_form("two passes")
     z.rk4_step(dt, ua, un, k)
+    z.set_rhs_form("one kernel")
     del un, k
     work = z.make_step_work()
     z.rk4_step_fused(dt, ub, work)

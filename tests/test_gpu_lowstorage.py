@@ -72,7 +72,7 @@ def test_ls_step_against_oracle_two_blocks(name):
 
 def test_ls_step_sommerfeld_faces():
     """Sommerfeld faces: the stage reads neighbouring values of its input, so
-    the fused step alternates two state buffers; equal to the stage
+    the fused step alternates two state buffers in either form; equal to the stage
     sequence and to the oracle with Z4cBoundaryRHS on the flagged faces."""
     faces = 0b101101  # ix1, ix2, ox2, ox3
     flags = [bool(faces >> f & 1) for f in range(6)]

@@ -385,9 +385,8 @@ def _uneven_batch(faces=True):
 def test_fused_step_equals_stage_sequence(cowling, faces):
     """z4c_rk4_step (RHS assembly + SumBT + AlgConstr fused per stage, ghosts
     at u_n) against four z4c_rk4_stage calls, over two steps, on a batch of
-    uneven blocks: the same sums in the same order.  With Sommerfeld faces
-    the stage states go through the two work registers; without, every stage
-    overwrites the state in place."""
+    uneven blocks: the same sums in the same order.  The stage sequence forms
+    its right-hand sides in two passes, the fused step in one kernel."""
     gs = _uneven_batch(faces)
     p = Params(**MP_GAUGE, cowling=cowling)
     host = [constrained_state(g, p, seed=20 + b) for b, g in enumerate(gs)]
@@ -399,7 +398,9 @@ def test_fused_step_equals_stage_sequence(cowling, faces):
     work = z.make_step_work()
     z.PrepareZ4cDerivatives(ua)
     for _ in range(2):
+        z.set_rhs_form("two passes")
         z.rk4_step(dt, ua, un, k)
+        z.set_rhs_form("one kernel")
         z.rk4_step_fused(dt, ub, work)
     torch.cuda.synchronize()
     A, Bf = z.download(ua, 22), z.download(ub, 22)
