@@ -27,7 +27,10 @@ def _batch(faces=0):
 @pytest.mark.parametrize("params", [
     dict(diss=0.02, damp_kappa1=0.02),
     dict(diss=0.1, damp_kappa1=0.3, damp_kappa2=0.2, chi_psi_power=-2.5, lapse_harmonic=0.7,
-         lapse_K=0.3, shift_alpha2Gamma=0.4, shift_H=0.2, lapse_advect=0.5, shift_advect=0.25)])
+         lapse_K=0.3, shift_alpha2Gamma=0.4, shift_H=0.2, lapse_advect=0.5, shift_advect=0.25),
+    # chi below its floor on most vertices, harmonic slicing, no shift driver
+    dict(diss=0.5, damp_kappa1=0.05, chi_div_floor=1.001, lapse_oplog=0.0, lapse_harmonic=1.0,
+         lapse_advect=0.0, shift_Gamma=0.0, shift_eta=0.0, shift_advect=0.0)])
 @pytest.mark.parametrize("matter", [False, True])
 def test_one_kernel_equals_two_passes(params, matter):
     gs = _batch()
