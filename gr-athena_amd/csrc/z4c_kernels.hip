@@ -3402,6 +3402,16 @@ int ensure_slots(z4c_ctx* c) {
   return Z4C_OK;
 }
 
+// Whether to run in two passes where the estimate (`two`) or z4c_set_rhs_form says
+// so: only a form that the caller fixed fails for want of memory, the estimate's
+// falls back to the one kernel, which needs no slots, for good.
+bool with_slots(z4c_ctx* c, bool two) {
+  if (!two || c->form || ensure_slots(c) == Z4C_OK) return two;
+  (void)hipGetLastError();
+  c->t_two = std::numeric_limits<double>::infinity();
+  return false;
+}
+
 // Bricks of the one-kernel right-hand side, cut as equal as they divide, and the
 // time of both forms.
 //
@@ -3453,7 +3463,8 @@ int build_fused_tiles(z4c_ctx* c, const std::vector<DevBlock>& hb) {
   const double lat = 20.0 + 1.75 * planes - (wgs >= 8 * NVAR ? 4.0 : 0.0);
   const double thr = 12.0 + 0.003 * wgs + 0.003 * march + 0.1 * alg;
   c->t_two = std::sqrt(std::sqrt(lat * lat * lat * lat + thr * thr * thr * thr));
-  return rhs_two(c) || step_two(c) ? ensure_slots(c) : Z4C_OK;
+  with_slots(c, rhs_two(c) || step_two(c));
+  return Z4C_OK;
 }
 
 // The launch does the work of the stencil and the assembly passes: the kernel
@@ -3511,7 +3522,7 @@ int launch_rhs(z4c_ctx* c, const z4c_params* p, const double* u,
   // side is written over its own input (every brick reads its neighbours' vertices)
   const long long nn = c->total_pts * NVAR;
   const bool apart = (uintptr_t)rhs + 8 * nn <= (uintptr_t)u || (uintptr_t)u + 8 * nn <= (uintptr_t)rhs;
-  if (apart && !rhs_two(c)) {
+  if (apart && !with_slots(c, rhs_two(c))) {
     FusedArgs a{};
     a.u = u;
     a.mat = mat;
@@ -5445,7 +5456,7 @@ int launch_rk4_step(z4c_ctx* c, const z4c_params* p, double dt, double* u, doubl
   // ghosts until the last stage.  In two passes without Sommerfeld faces every
   // stage state overwrites u's interior (u_n is kept in W1 as well), and a ghost
   // update finds u_n's ghosts in W0.
-  const bool two = p->cowling || step_two(c);
+  const bool two = p->cowling || with_slots(c, step_two(c));
   const bool inplace = two && !c->faces;
   const bool held = !ghosts || inplace;  // u_n kept in W1, not in u
   double* const outs[4] = {inplace ? u : W0, held ? u : W1, inplace ? u : W0, u};
@@ -5550,7 +5561,7 @@ int launch_ls_step(z4c_ctx* c, const z4c_params* p, const z4c_ls_tableau* T, dou
     if (ghosts && !all_ghosts) extra += (T->nstages - odd) * 0.026 * c->ntiles[BOX_GHOST];
     extra /= T->nstages;
   }
-  const bool two = p->cowling || step_two(c, extra);
+  const bool two = p->cowling || with_slots(c, step_two(c, extra));
   const bool inplace = two && !c->faces;
   double* cur = u;
   int rc = Z4C_OK;
