@@ -3377,11 +3377,11 @@ void launch_stencil_cfg(int cfg, const StencilArgs& sa, hipStream_t s) {
   }
 }
 
-// Whether z4c_rhs runs in two passes, and the stages of a step: a stage in one
-// kernel pays for the second buffer that its state goes to, about 5 % of a
-// right-hand side, and `extra` us.
+// Whether z4c_rhs runs in two passes (3 % in doubt: the one kernel, which needs no
+// slots), and the stages of a step: a stage in one kernel pays for the second
+// buffer that its state goes to, about 5 % of a right-hand side, and `extra` us.
 bool rhs_two(const z4c_ctx* c) {
-  return c->form ? c->form == Z4C_FORM_TWO_PASSES : c->t_one >= c->t_two;
+  return c->form ? c->form == Z4C_FORM_TWO_PASSES : c->t_one >= 1.03 * c->t_two;
 }
 bool step_two(const z4c_ctx* c, double extra = 0.0) {
   return c->form ? c->form == Z4C_FORM_TWO_PASSES : c->t_one + extra >= 0.95 * c->t_two;
@@ -3417,18 +3417,18 @@ bool with_slots(z4c_ctx* c, bool two) {
 //
 // One kernel: a brick takes 35 to 37 us however few there are (its 22 fields in
 // turn), 53 us with a second one on its CU, 84 us when a third round begins, and
-// from there 0.0955 us a brick.  Two passes: a workgroup of the stencil pass
+// from there 0.093 us a brick.  Two passes: a workgroup of the stencil pass
 // marches the planes of a tile, 1.75 us each on top of 20 us (16 us once there
 // are enough for the fields of a tile to meet on one XCD); a full chip takes
 // 0.003 us a workgroup and 0.003 us a plane, the algebra 0.1 us per 256 vertices.
 // Tiles that split a block's rows take half as long again a plane.  Against 132
 // batches measured in both forms (2 to 64 cells a side; cubes, rods, plates and
-// mixtures; 1 to 2048 blocks) the first estimate is within 5 % (rms) and the
-// second within 9 % (7 % where the two are close).  z4c_rhs in the form that they
-// favour loses 0.3 % to the better one on average and 11 % at most (64 blocks of
-// 2^3 cells, 38.0 against 34.0 us); always one kernel loses 4.4 % on average and
-// up to 58 % (16 blocks of 2^3: 34.0 against 21.5 us; 64 of 4 x 64 x 4: 160
-// against 105).
+// mixtures; 1 to 2048 blocks) the first estimate is within 6 % (rms) and the
+// second within 9 % (7 % where the two are close).  z4c_rhs in the form that
+// rhs_two takes from them loses 0.12 % to the better one on average and 4 % at most
+// (18 blocks of 15 x 24 x 3 cells, 39.7 against 38.1 us), an rk4 step 0.11 % and 4 %;
+// always one kernel loses 4.4 % on average and up to 58 % (16 blocks of 2^3: 34.0
+// against 21.5 us; 64 of 4 x 64 x 4: 160 against 105).
 int build_fused_tiles(z4c_ctx* c, const std::vector<DevBlock>& hb) {
   constexpr int M[3] = {FuCfg::BX, FuCfg::BY, FuCfg::BZ};
   std::vector<FusedTile> t;
@@ -3459,7 +3459,7 @@ int build_fused_tiles(z4c_ctx* c, const std::vector<DevBlock>& hb) {
   HIPCALL(hipMemcpy(c->fu_tiles, t.data(), sizeof(FusedTile) * t.size(), hipMemcpyHostToDevice));
   c->fu_ntiles = (int)t.size();
   const double nt = (double)t.size(), cu = c->n_cu;
-  c->t_one = std::max(nt > 2 * cu ? 84.0 : nt > cu ? 53.0 : 37.0, 0.0955 * nt + 8.0);
+  c->t_one = std::max(nt > 2 * cu ? 84.0 : nt > cu ? 53.0 : 37.0, 0.093 * nt + 8.0);
   const double lat = 20.0 + 1.75 * planes - (wgs >= 8 * NVAR ? 4.0 : 0.0);
   const double thr = 12.0 + 0.003 * wgs + 0.003 * march + 0.1 * alg;
   c->t_two = std::sqrt(std::sqrt(lat * lat * lat * lat + thr * thr * thr * thr));
